@@ -1,0 +1,78 @@
+"""The 256-row tile of the tiled expert GEMMs at its edges: experts that end on
+either side of every 64-row part, and step counts of every remainder modulo the
+five operand buffers its K loop rotates through (and fewer steps than buffers).
+
+Every product is compared with float64 torch on the same 16-bit operands.  A
+GEMM sums K terms in fp32 (relative error at most K 2^-24 of the sum of the
+magnitudes); h is then rounded to 16 bits (2^-9 relative in bf16), y is not.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+COUNTS = [1, 63, 64, 65, 128, 129, 192, 193, 255, 256, 257, 321]
+
+
+def _layout(dev, g):
+    offsets, tiles = [0], []
+    for k, c in enumerate(COUNTS):
+        tiles += [[k, offsets[k] + r0, min(64, c - r0), 0] for r0 in range(0, c, 64)]
+        offsets.append(offsets[-1] + c)
+    slots = torch.randperm(offsets[-1], generator=g).to(torch.int32)
+    as_dev = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    return offsets, slots, as_dev(offsets), slots.to(dev), as_dev(tiles), len(tiles)
+
+
+@pytest.mark.parametrize("steps", [1, 4, 5, 6, 7, 8, 9])
+def test_tile256_gemms_match_float64(steps):
+    from treemoe_spec_amd import _capi
+
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(steps)
+    e, rows = len(COUNTS), sum(COUNTS)
+    t, h, i = rows // 2, 64 * steps, 256
+    assert rows % 2 == 0 and rows >= 112 * e      # the 256-row tile's rule
+    print(f"tile256 steps={steps}", flush=True)
+    offsets, slots, off_d, slots_d, tiles_d, nt = _layout(dev, g)
+    draw = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    x, w1, w3 = draw(t, h), draw(e, i, h) * 0.1, draw(e, i, h) * 0.1
+    xd, w1d, w3d = x.to(dev), w1.to(dev), w3.to(dev)
+    hd = torch.full((rows + 1, i), 7.0, dtype=torch.bfloat16, device=dev)
+    st = _capi.stream_of(dev)
+    _capi.call("tm_op1_prefill_gemm1", xd.data_ptr(), w1d.data_ptr(), w3d.data_ptr(),
+               hd.data_ptr(), slots_d.data_ptr(), off_d.data_ptr(), tiles_d.data_ptr(), nt, t, h,
+               i, e, _capi.TM_DTYPE_BF16, st)
+    out = hd.double().cpu()
+    assert torch.all(out[rows] == 7.0)
+    for k in range(e):
+        r = slice(offsets[k], offsets[k + 1])
+        xf = x[slots[r].long() >> 1].double()
+        a, b = xf @ w1[k].double().T, xf @ w3[k].double().T
+        ref = a * torch.sigmoid(a) * b
+        # one bf16 rounding, plus the fp32 sums' share where a and b cancel
+        tol = 2.0 ** -8 * ref.abs() + 1e-5 * (1.0 + a.abs()) * (1.0 + b.abs())
+        assert torch.all((out[r] - ref).abs() <= tol), (steps, COUNTS[k])
+
+    # down: K = 64 * steps per segment, two segments, H = 256
+    ki, n = 128 * steps, 256
+    hm, w2 = draw(rows, ki), draw(e, n, ki) * 0.1
+    gates = torch.rand(rows, generator=g)
+    hmd, w2d, gd = hm.to(dev), w2.to(dev), gates.to(dev)
+    y = torch.full((2, rows, n), 7.0, device=dev)
+    _capi.call("tm_op1_prefill_gemm2", hmd.data_ptr(), w2d.data_ptr(), y.data_ptr(),
+               gd.data_ptr(), slots_d.data_ptr(), off_d.data_ptr(), tiles_d.data_ptr(), nt, 2, t,
+               n, ki, e, _capi.TM_DTYPE_BF16, st)
+    out = y.double().cpu()
+    half = ki // 2
+    for k in range(e):
+        r = slice(offsets[k], offsets[k + 1])
+        for s in range(2):
+            a, w = hm[r, s * half:(s + 1) * half].double(), w2[k, :, s * half:(s + 1) * half].double()
+            gate = gates[slots[r].long()].double()[:, None]
+            ref, mag = gate * (a @ w.T), gate * (a.abs() @ w.abs().T)
+            tol = (half + 2) * 2.0 ** -24 * mag
+            assert torch.all((out[s, r] - ref).abs() <= tol), (steps, COUNTS[k], s)

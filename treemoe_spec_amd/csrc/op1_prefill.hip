@@ -5,35 +5,29 @@
 // wrong shape.  These kernels tile both operands:
 //
 //   workgroup = NW waves (2 row halves x NW / 2 column groups) = BM sorted rows
-//   x 32 NW weight rows; each wave owns BM/2 x 64 outputs = (BM/64) x 2
-//   v_mfma_f32_32x32x16_bf16 tiles (on gfx950 the 32x32 form sustains ~2.2
+//   x BN weight rows; each wave owns BM/2 x 32 NJ outputs = (BM/64) x NJ
+//   v_mfma_f32_32x32x16 tiles (on gfx950 the 32x32 form sustains ~2.2
 //   PFLOP/s, the 16x16x32 form ~1.3).
 //   Operands go from global memory straight into LDS (16-byte buffer loads
 //   with the LDS flag: lane i of a load lands at byte 16 i of its 1 KB block,
-//   no registers involved), NS stages deep: while the MFMAs of step k run,
-//   steps k+1 .. k+NS-1 are in flight.  LDS rows hold one K step (2 BK bytes)
-//   with the 16-byte chunks XOR-swizzled (swz), which the loads arrange by
-//   choosing each lane's source chunk; 16 consecutive rows read at one
-//   logical chunk then hit 16 distinct 4-bank groups.
+//   no registers involved), several steps deep.  LDS rows hold one K step of
+//   64 (128 bytes: a whole cache line per row and load) with the 16-byte chunks
+//   XOR-swizzled (swz), which the loads arrange by choosing each lane's source
+//   chunk; 16 consecutive rows read at one logical chunk then hit 16 distinct
+//   4-bank groups.
 //
-// Three tile configurations, all 8 waves x 256 weight rows but the last:
-// BM = 128 with K steps of 64 and three 48 KB stages; BM = 256 with K steps
-// of 32 and four 32 KB stages (fewer operand bytes per flop, larger jobs);
-// BM = 64 with K steps of 64 against 128 weight rows on 4 waves, three 24 KB
-// stages, so two workgroups share a CU.  Down always uses the first; gate/up
-// uses the second when the experts average 384 rows or more and the third
-// when the tile list leaves at most 16 rows per entry.  A tile whose M-tile
-// holds fewer than BM real rows runs the MFMAs of the 64-row parts that hold
-// them only.  Where the MFMAs bound the kernel (the 256-row gate/up tile, and
-// the down GEMM when the experts average 384 rows or more) the two 4-wave
-// halves of a workgroup run the K loop half a step apart (k_loop_pp), so one
-// wave per SIMD issues MFMAs while the other reads its fragments (config 5,
-// same box: gate/up 1045 -> 990 us, down 576 -> 558 us, bit-identical).
+// Three tile configurations:
+//   Tile256  256 rows x 256 weight rows on 4 waves, one per SIMD, hand-
+//            pipelined (PipeLoop): where the experts average 112 rows or more;
+//   Tile128  128 x 256 on 8 waves, three 48 KB stages;
+//   TileDec  64 x 128 on 4 waves, three 24 KB stages, so two workgroups share
+//            a CU: gate/up when the tile list leaves at most 16 rows per entry.
+// A tile whose M-tile holds fewer than BM real rows runs the MFMAs of the
+// 64-row parts that hold them only.
 //
-// Gate/up: B = 128 rows of w1 and the same 128 rows of w3 (64 and 64 in the
-// 4-wave tile), so each wave holds the gate and up sums of the same outputs
-// and applies SwiGLU in registers; h is written row-major [sorted row, I]
-// through an LDS-staged, coalesced store.
+// Gate/up: B = BN / 2 rows of w1 and the same rows of w3, so each wave holds
+// the gate and up sums of the same outputs and applies SwiGLU in registers; h
+// is written row-major [sorted row, I] through an LDS-staged, coalesced store.
 // Down: B = 256 rows of w2 over one K segment; the gate weight multiplies the
 // fp32 sums before the store of the partial y[segment].
 //
@@ -56,17 +50,16 @@ constexpr uint32_t kOOR = 0x80000000u;   // out-of-range buffer offset: loads 0
 
 // Tile configuration: BM sorted rows per M-tile, K steps of BK, NS stages,
 // BN weight rows per workgroup, NTH threads (NTH / 64 waves as 2 row halves x
-// NTH / 128 column groups of 32 outputs, so BN = 32 x waves).
-template <int BM, int BK, int NS, int BN = 256, int NTH = 512, bool PINGPONG = false>
+// NTH / 128 column groups; a wave owns BM/2 x 32 NJ outputs).
+template <int BM, int BK, int NS, int BN = 256, int NTH = 512>
 struct Tile {
-  // the two wave halves run the K loop half a step apart (k_loop_pp)
-  static constexpr bool PP = PINGPONG;
   static constexpr int PBM = BM;
   static constexpr int PBK = BK;
   static constexpr int NSTAGE = NS;
   static constexpr int PBN = BN;                  // weight rows per workgroup
   static constexpr int NT = NTH;                  // threads per workgroup
   static constexpr int NW = NTH / 64;             // waves
+  static constexpr int NJ = BN / (16 * NW);       // 32-column accumulator tiles per wave
   static constexpr int PROW = PBK * 2;            // LDS row, bytes (PROW / 16 swizzled chunks)
   static constexpr int CPR = PROW / 16;           // 16-byte chunks per row
   static constexpr int RPB = 256 / PROW;          // rows per 256 B (one pass over the 64 banks)
@@ -78,25 +71,23 @@ struct Tile {
   static constexpr int BLD = BBYTES / (NT * 16);  //                                   B
   static constexpr int LDS_PER_STEP = ALD + BLD;
   static constexpr int MT = PBM / 64;             // 32-row accumulator tiles per wave
-  // weight loads of an expert with a single M-tile go non-temporal (below)
-  // for tiles of at most 128 rows; the 256-row gate/up tile runs where most
-  // experts take several M-tiles, and there the policy measured slower
-  static constexpr bool NT_WEIGHTS = BM <= 128;
-  // bf16 h staging: rows of PBN / 2 columns, padded by 16 bytes; rows per
-  // stage: the whole tile in one stage when it fits
+  // one wave per SIMD; A and B tiles in a ring of NS buffers (k_loop_pipe)
+  static constexpr bool PIPE = NJ == 4;
+  static constexpr int BUF = PIPE ? ABYTES : STAGE;  // one LDS buffer
+  // h staging: rows of PBN / 2 columns, padded by 16 bytes; rows per stage:
+  // the whole tile in one stage when it fits
   static constexpr int HSTRIDE = PBN + 16;
-  static constexpr int HROWS = PBM * HSTRIDE <= STAGE ? PBM : PBM / NSTAGE;
+  static constexpr int HROWS = PBM * HSTRIDE <= BUF ? PBM : PBM / 4;
   static_assert(ALD >= 1 && BLD >= 1 && BLD % 2 == 0 && CPR >= 4, "tile shape");
-  static_assert(PBN == 32 * NW && (NW == 4 || NW == 8), "wave layout");
-  static_assert(NS == 3 || NS == 4, "stage rotation");
-  static_assert(HROWS * HSTRIDE <= STAGE && (PBM + HROWS - 1) / HROWS <= NS, "h staging");
-  static_assert(NS * STAGE <= 160 * 1024, "LDS");
-  static_assert(!PINGPONG || NTH == 512, "ping-pong: two halves of four waves");
+  static_assert((NJ == 2 || NJ == 4) && (NW == 4 || NW == 8), "wave layout");
+  static_assert(NS == (PIPE ? 5 : 3), "buffer rotation");
+  static_assert(HROWS * HSTRIDE <= BUF && (PBM + HROWS - 1) / HROWS <= NS, "h staging");
+  static_assert(NS * BUF <= 160 * 1024, "LDS");
+  static_assert(!PIPE || (PBK == 64 && ABYTES == BBYTES), "k_loop_pipe's buffers");
 };
 using Tile128 = Tile<128, 64, 3>;
-using Tile256 = Tile<256, 32, 4, 256, 512, true>;
-// The down GEMM's tile where the experts average many rows (MFMA-bound).
-using Tile128PP = Tile<128, 64, 3, 256, 512, true>;
+// Many rows per expert: 256 x 256 on four waves of 128 x 128 outputs.
+using Tile256 = Tile<256, 64, 5, 256, 256>;
 // Few rows per expert: 64-row M-tiles against 128 weight rows with 4 waves,
 // 72 KB of LDS, so two workgroups share a CU.  Same per-output K order as
 // Tile128, so the same bits.
@@ -111,21 +102,38 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t pbuf(const void* base, uint32_
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
-// 32x32x16 bf16 MFMA.  Lane l: A row l % 32 and B column l % 32, k 8 (l / 32)
-// .. +7; accumulator value v is C[8 (v / 4) + 4 (l / 32) + v % 4][l % 32].
-// (DT: TM_DTYPE_BF16 or TM_DTYPE_F16 operands, same lane layout.)
+// 32x32x16 MFMA with the weights as the first operand: x holds 32 sorted rows
+// and w 32 weight rows (lane l: row l % 32, k 8 (l / 32) .. +7), and lane l gets
+// C[row l % 32][column 8 (v / 4) + 4 (l / 32) + v % 4] in accumulator value v,
+// so its values 4 q .. 4 q + 3 are four consecutive output columns of one row
+// (acc_col): the epilogues pack and store them as one vector.  (DT:
+// TM_DTYPE_BF16 or TM_DTYPE_F16 operands, same lane layout.)
 template <int DT>
-__device__ __forceinline__ f32x16_t pmfma(u32x4_t a, u32x4_t b, f32x16_t c) {
+__device__ __forceinline__ f32x16_t pmfma(u32x4_t x, u32x4_t w, f32x16_t c) {
   if constexpr (DT == TM_DTYPE_F16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
-                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, w),
+                                                  __builtin_bit_cast(f16x8_t, x), c, 0, 0, 0);
   else
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, w),
+                                                   __builtin_bit_cast(bf16x8_t, x), c, 0, 0, 0);
 }
 
-__device__ __forceinline__ int acc_row(int v, int lane) {
-  return 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+// First of the four output columns that accumulator values 4 q .. 4 q + 3 hold.
+__device__ __forceinline__ int acc_col(int q, int lane) { return 8 * q + 4 * (lane >> 5); }
+
+// Four fp32 values to the 16-bit type, round to nearest even, packed in order
+// (bf16: v_cvt_pk_bf16_f32, one instruction per pair).
+typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+template <int DT>
+__device__ __forceinline__ uint32_t pack16(float lo, float hi) {
+  const f32x2_t v = {lo, hi};
+  if constexpr (DT == TM_DTYPE_F16)
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
+  else
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
 }
 
 // Byte offset in a swizzled tile of logical chunk c (16 B) of row r: chunk c
@@ -166,11 +174,20 @@ __device__ __forceinline__ bool job_of(int L, int n_mt, int ncol, int* mt, int* 
   return *col < ncol;
 }
 
-// Job of launch index L for the prefill GEMMs: M-tile (in the compact
-// expert-major order) and column job, or false for a launch index past the
-// real jobs (those are the launch's last indices).  The first wave scans
-// ceil(rows_e / BM) over the experts (E <= 64 loads).  When the active
-// experts average two M-tiles or more, XCD x = L % 8 walks its column jobs
+// One workgroup's job: rows p0 .. p0 + rows of expert e against column job
+// col; single: the expert's only M-tile.
+struct Job {
+  int e, p0, rows, col;
+  bool single;
+};
+
+// Job of launch index L for the prefill GEMMs, or false for a launch index
+// past the real jobs (those are the launch's last indices).  Lane e of every
+// wave holds expert e's row count (no LDS, no barrier); wave scans of
+// ceil(rows_e / BM) and ceil(rows_e / 64) give the M-tiles and the 64-row tiles
+// before each expert, so the owner of M-tile m is found with a ballot instead
+// of a loop of dependent loads over the experts.  When the active experts
+// average two M-tiles or more, XCD x = L % 8 walks its column jobs
 // [x * cpx, (x + 1) * cpx) of every M-tile one expert at a time, the
 // expert's M-tiles fastest, then its columns: the ~32 workgroups resident on
 // an XCD then run the jobs of one expert or of a few adjacent ones, so all
@@ -182,23 +199,31 @@ __device__ __forceinline__ bool job_of(int L, int n_mt, int ncol, int* mt, int* 
 // against 1771, T = 4096 3111 against 3202, T = 1536 1374 against 1411; but
 // T = 128 535 against 501, T = 256 542 against 513, T = 512 720 against 705,
 // where most experts take one M-tile.)
+// An expert whose first entry in the 64-row tile list is masked (expert -1,
+// as Routing.exclude_experts leaves it) has no jobs, like the weight-streaming
+// kernels skip its tiles.
 template <class C>
-__device__ __forceinline__ bool expert_job(int L, const int32_t* __restrict__ offsets, int E,
-                                           int mt_max, int ncol, int* mt, int* col) {
-  // every wave computes the job itself (no LDS, no barrier)
+__device__ __forceinline__ bool expert_job(int L, const int32_t* __restrict__ offsets,
+                                           const int32_t* __restrict__ tiles, int max_tiles,
+                                           int E, int mt_max, int ncol, Job* job) {
   const int x = L % kXcds, l = L / kXcds;
   const int cpx = (ncol + kXcds - 1) / kXcds;
   const int lane = threadIdx.x & 63;
-  int n = 0;
+  int off = 0, cnt = 0;
   if (lane < E) {
-    const int cnt = offsets[lane + 1] - offsets[lane];
-    n = (cnt + C::PBM - 1) / C::PBM;
+    off = offsets[lane];
+    cnt = offsets[lane + 1] - off;
   }
-  int incl = n;
+  const int n = (cnt + C::PBM - 1) / C::PBM;
+  const int n64 = (cnt + TM_GEMM_TILE_M - 1) / TM_GEMM_TILE_M;
+  int incl = n, incl64 = n64;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
-    const int t = __shfl_up(incl, o);
-    if (lane >= o) incl += t;
+    const int t = __shfl_up(incl, o), t64 = __shfl_up(incl64, o);
+    if (lane >= o) {
+      incl += t;
+      incl64 += t64;
+    }
   }
   const int first = incl - n;  // M-tiles of the experts before this lane's
   const int total = __shfl(incl, 63);
@@ -222,43 +247,25 @@ __device__ __forceinline__ bool expert_job(int L, const int32_t* __restrict__ of
       c = __shfl(x * cpx + (n > 0 ? j / n : 0), src);
     }
   }
-  *mt = __builtin_amdgcn_readfirstlane(m);
-  *col = __builtin_amdgcn_readfirstlane(c);
-  return *mt >= 0 && *mt < mt_max && *col < ncol;
+  m = __builtin_amdgcn_readfirstlane(m);
+  job->col = __builtin_amdgcn_readfirstlane(c);
+  if (m < 0 || m >= mt_max || job->col >= ncol) return false;
+  const unsigned long long own = __ballot(m >= first && m < incl);
+  if (own == 0ull) return false;
+  const int e = __ffsll((long long)own) - 1;
+  const int tile64 = __builtin_amdgcn_readlane(incl64 - n64, e);
+  if (tile64 >= max_tiles || tiles[4 * tile64] != e) return false;
+  const int m0 = (m - __builtin_amdgcn_readlane(first, e)) * C::PBM;
+  job->e = e;
+  job->p0 = __builtin_amdgcn_readlane(off, e) + m0;
+  job->rows = min(C::PBM, __builtin_amdgcn_readlane(cnt, e) - m0);
+  job->single = __builtin_amdgcn_readlane(n, e) == 1;
+  return true;
 }
 
 // Launch size: 8 XCDs x (M-tile bound) x the columns of one XCD's range.
 int64_t launch_jobs(int64_t mt_max, int64_t ncol) {
   return kXcds * mt_max * ((ncol + kXcds - 1) / kXcds);
-}
-
-// M-tile `idx` of the compact expert-major order: expert, first row, rows.
-// An expert whose first entry in the 64-row tile list is masked (expert -1,
-// as Routing.exclude_experts leaves it) is skipped, like the weight-streaming
-// kernels skip its tiles.
-template <class C>
-__device__ __forceinline__ bool find_mtile(const int32_t* __restrict__ offsets,
-                                           const int32_t* __restrict__ tiles, int max_tiles,
-                                           int E, int idx, int* e, int* p0, int* rows,
-                                           bool* single) {
-  int acc = 0, tile64 = 0;
-  for (int k = 0; k < E; ++k) {
-    const int o = offsets[k];
-    const int cnt = offsets[k + 1] - o;
-    const int nt = (cnt + C::PBM - 1) / C::PBM;
-    if (idx < acc + nt) {
-      if (tile64 >= max_tiles || tiles[4 * tile64] != k) return false;
-      const int m0 = (idx - acc) * C::PBM;
-      *e = k;
-      *p0 = o + m0;
-      *rows = min(C::PBM, cnt - m0);
-      *single = nt == 1;
-      return true;
-    }
-    acc += nt;
-    tile64 += (cnt + TM_GEMM_TILE_M - 1) / TM_GEMM_TILE_M;
-  }
-  return false;
 }
 
 // Upper bound of the M-tiles over E experts holding `slots` rows.
@@ -273,8 +280,9 @@ int64_t mtile_bound(int64_t slots, int64_t E) {
 // l % CPR, so it fetches the logical chunk that the swizzle stores there.
 template <class C>
 struct DmaLoad {
-  __amdgpu_buffer_rsrc_t ra;        // A
-  __amdgpu_buffer_rsrc_t rb0, rb1;  // B: the first and the second half of its loads
+  const void* pa;         // A
+  const void *pb0, *pb1;  // B: the first and the second half of its loads
+  uint32_t na, nb;        // bytes behind pa, and behind each of pb0 and pb1
   uint32_t aoff[C::ALD];  // byte offset of the chunk at k = 0, or kOOR
   uint32_t boff[C::BLD];
 };
@@ -289,41 +297,47 @@ __device__ __forceinline__ int dma_chunk(int row) {
   return (threadIdx.x & (C::CPR - 1)) ^ ((row / C::RPB) & (C::CPR - 1));
 }
 
-// Step `kstep` (K bytes PROW kstep ..) of both tiles into `st`: the A loads,
-// then the B loads; past the end of K the loads are out of range and store
-// zeros.  Every step issues all LDS_PER_STEP loads in this order, so the wait
-// counts below stay exact.  (Spreading a step's loads between the previous
-// step's MFMAs instead measured no faster.)
 // One 16-byte buffer load per lane into LDS at `lds` + 16 lane (lds
-// wave-uniform).  A plain function: the host compilation pass rejects the
-// builtin inside some instantiations of the templates below.
+// wave-uniform), from byte voffset (per lane) + soffset (wave-uniform).  A
+// plain function: the host compilation pass rejects the builtin inside some
+// instantiations of the templates below.
 __device__ __forceinline__ void lds_load16(__amdgpu_buffer_rsrc_t r, uint8_t* lds,
-                                           uint32_t voffset) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, voffset, 0, 0, 0);
+                                           uint32_t voffset, uint32_t soffset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, voffset, soffset, 0, 0);
 }
 // The same with the non-temporal cache policy (weights streamed through).
 __device__ __forceinline__ void lds_load16_nt(__amdgpu_buffer_rsrc_t r, uint8_t* lds,
-                                              uint32_t voffset) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, voffset, 0, 0, 2);
+                                              uint32_t voffset, uint32_t soffset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, voffset, soffset, 0, 2);
 }
 
+// Load i of step `kstep` (K bytes PROW kstep ..) of the A tile into `at` or of
+// the B tile into `bt`.  The K position is the load's scalar offset, so a step costs no
+// vector arithmetic; past the end of K the buffer has no bytes, so the load
+// is out of range and stores zeros without memory traffic.  Every step issues
+// all LDS_PER_STEP loads, so the wait counts below stay exact.
+template <class C>
+__device__ __forceinline__ void dma_a(const DmaLoad<C>& d, uint8_t* at, int i, int kstep, int nk) {
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // LDS base: wave-uniform
+  lds_load16(pbuf(d.pa, kstep < nk ? d.na : 0u), at + (C::NW * i + w) * 1024, d.aoff[i],
+             (uint32_t)kstep * (uint32_t)C::PROW);
+}
+template <class C, bool NTB>
+__device__ __forceinline__ void dma_b(const DmaLoad<C>& d, uint8_t* bt, int i, int kstep, int nk) {
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const __amdgpu_buffer_rsrc_t r = pbuf(i < C::BLD / 2 ? d.pb0 : d.pb1, kstep < nk ? d.nb : 0u);
+  uint8_t* const lds = bt + (C::NW * i + w) * 1024;
+  if constexpr (NTB)
+    lds_load16_nt(r, lds, d.boff[i], (uint32_t)kstep * (uint32_t)C::PROW);
+  else
+    lds_load16(r, lds, d.boff[i], (uint32_t)kstep * (uint32_t)C::PROW);
+}
 template <class C, bool NTB>
 __device__ __forceinline__ void dma_step(const DmaLoad<C>& d, uint8_t* st, int kstep, int nk) {
-  const uint32_t kb = (uint32_t)kstep * (uint32_t)C::PROW;
-  const bool valid = kstep < nk;
-  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // LDS base: wave-uniform
 #pragma unroll
-  for (int i = 0; i < C::ALD; ++i)
-    lds_load16(d.ra, st + (C::NW * i + w) * 1024,
-               (valid && d.aoff[i] != kOOR) ? d.aoff[i] + kb : kOOR);
+  for (int i = 0; i < C::ALD; ++i) dma_a<C>(d, st, i, kstep, nk);
 #pragma unroll
-  for (int i = 0; i < C::BLD; ++i)
-    if constexpr (NTB)
-      lds_load16_nt(i < C::BLD / 2 ? d.rb0 : d.rb1, st + C::ABYTES + (C::NW * i + w) * 1024,
-                    valid ? d.boff[i] + kb : kOOR);
-    else
-      lds_load16(i < C::BLD / 2 ? d.rb0 : d.rb1, st + C::ABYTES + (C::NW * i + w) * 1024,
-                 valid ? d.boff[i] + kb : kOOR);
+  for (int i = 0; i < C::BLD; ++i) dma_b<C, NTB>(d, st + C::ABYTES, i, kstep, nk);
 }
 
 // Wait until at most n of this thread's vector-memory operations are
@@ -346,179 +360,226 @@ __device__ __forceinline__ u32x4_t frag(const uint8_t* tile, int row, int s, int
 // whole M-tile, a smaller M its first 64 M rows (a tile with at most 64 M real
 // rows, whose other rows are zeros).
 template <class C, int M, int DT>
-__device__ __forceinline__ void compute_step(const uint8_t* st, const int (&brow)[2],
-                                             f32x16_t (&acc)[M][2]) {
+__device__ __forceinline__ void compute_step(const uint8_t* st, const int (&brow)[C::NJ],
+                                             f32x16_t (&acc)[M][C::NJ]) {
   const int lane = threadIdx.x & 63;
   const int wm = (threadIdx.x >> 6) & 1;
   constexpr int S = C::PBK / 16;
-  if constexpr (S >= 4) {
-    // K steps of 64: the fragments of k-step s + 1 are read between the
-    // MFMAs of k-step s (one MFMA, then one LDS read, while reads remain), so
-    // each MFMA waits only for reads issued a k-step earlier.  Same MFMAs in
-    // the same order.  (Config 5 down GEMM 588 -> 569 us same-box; on the
-    // 256-row gate/up tile, whose steps have two k-steps, it measured slower,
-    // 1043 -> 1068 us, so that tile keeps the loop below.)
-    u32x4_t a[2][M], b[2][2];
+  // The fragments of k-step s + 1 are read between the MFMAs of k-step s (one
+  // MFMA, then one LDS read, while reads remain), so each MFMA waits only for
+  // reads issued a k-step earlier.
+  u32x4_t a[2][M], b[2][2];
 #pragma unroll
-    for (int i = 0; i < M; ++i) a[0][i] = frag<C>(st, 32 * M * wm + 32 * i, 0, lane);
+  for (int i = 0; i < M; ++i) a[0][i] = frag<C>(st, 32 * M * wm + 32 * i, 0, lane);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) b[0][j] = frag<C>(st + C::ABYTES, brow[j], 0, lane);
+  for (int j = 0; j < 2; ++j) b[0][j] = frag<C>(st + C::ABYTES, brow[j], 0, lane);
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      const int cur = s & 1, nxt = cur ^ 1;
-      __builtin_amdgcn_sched_barrier(0);
-      if (s + 1 < S) {
-#pragma unroll
-        for (int i = 0; i < M; ++i) a[nxt][i] = frag<C>(st, 32 * M * wm + 32 * i, s + 1, lane);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) b[nxt][j] = frag<C>(st + C::ABYTES, brow[j], s + 1, lane);
-      }
-#pragma unroll
-      for (int i = 0; i < M; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = pmfma<DT>(a[cur][i], b[cur][j], acc[i][j]);
-      if (s + 1 < S) {
-#pragma unroll
-        for (int k = 0; k < M + 2 && k < 2 * M; ++k) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
-        }
-        if constexpr (2 * M > M + 2)
-          __builtin_amdgcn_sched_group_barrier(0x008, 2 * M - (M + 2), 0);
-      }
-    }
-    // keep the next step's wait, barrier and loads after these MFMAs
+  for (int s = 0; s < S; ++s) {
+    const int cur = s & 1, nxt = cur ^ 1;
     __builtin_amdgcn_sched_barrier(0);
-  } else {
+    if (s + 1 < S) {
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      u32x4_t a[M], b[2];
+      for (int i = 0; i < M; ++i) a[nxt][i] = frag<C>(st, 32 * M * wm + 32 * i, s + 1, lane);
 #pragma unroll
-      for (int i = 0; i < M; ++i) a[i] = frag<C>(st, 32 * M * wm + 32 * i, s, lane);
+      for (int j = 0; j < 2; ++j) b[nxt][j] = frag<C>(st + C::ABYTES, brow[j], s + 1, lane);
+    }
 #pragma unroll
-      for (int j = 0; j < 2; ++j) b[j] = frag<C>(st + C::ABYTES, brow[j], s, lane);
+    for (int i = 0; i < M; ++i)
 #pragma unroll
-      for (int i = 0; i < M; ++i)
+      for (int j = 0; j < 2; ++j) acc[i][j] = pmfma<DT>(a[cur][i], b[cur][j], acc[i][j]);
+    if (s + 1 < S) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = pmfma<DT>(a[i], b[j], acc[i][j]);
+      for (int k = 0; k < M + 2 && k < 2 * M; ++k) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
+      }
+      if constexpr (2 * M > M + 2)
+        __builtin_amdgcn_sched_group_barrier(0x008, 2 * M - (M + 2), 0);
     }
   }
+  // keep the next step's wait, barrier and loads after these MFMAs
+  __builtin_amdgcn_sched_barrier(0);
 }
 
-// The LDS stages: distinct arrays used in a fixed rotation, so the compiler
-// can tell the stage being read from the ones being loaded (s3 is unused with
-// three stages).
+// The LDS buffers: distinct arrays used in a fixed rotation, so the compiler
+// can tell the one being read from the ones being loaded (s3 and s4 are used by
+// Tile256 only).
 struct Stages {
   uint8_t* s0;
   uint8_t* s1;
   uint8_t* s2;
   uint8_t* s3;
+  uint8_t* s4;
 };
+#define TM_STAGES(C)                                                                   \
+  __shared__ __attribute__((aligned(16))) uint8_t s0[C::BUF];                          \
+  __shared__ __attribute__((aligned(16))) uint8_t s1[C::BUF];                          \
+  __shared__ __attribute__((aligned(16))) uint8_t s2[C::BUF];                          \
+  __shared__ __attribute__((aligned(16))) uint8_t s3[C::NSTAGE > 3 ? C::BUF : 16];     \
+  __shared__ __attribute__((aligned(16))) uint8_t s4[C::NSTAGE > 4 ? C::BUF : 16];     \
+  const Stages sb{s0, s1, s2, s3, s4}
 
 // A workgroup barrier (after this wave's LDS operations) that the compiler
 // schedules nothing across.
-__device__ __forceinline__ void pp_barrier() {
+__device__ __forceinline__ void step_barrier() {
   __builtin_amdgcn_sched_barrier(0);
   tm_lds_barrier();
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// All fragments of one staged step (S = BK / 16 k-steps) into registers.
-template <class C, int M>
-__device__ __forceinline__ void read_step(const uint8_t* st, const int (&brow)[2],
-                                          u32x4_t (&a)[C::PBK / 16][M],
-                                          u32x4_t (&b)[C::PBK / 16][2]) {
-  const int lane = threadIdx.x & 63;
-  const int wm = (threadIdx.x >> 6) & 1;
-#pragma unroll
-  for (int s = 0; s < C::PBK / 16; ++s) {
-#pragma unroll
-    for (int i = 0; i < M; ++i) a[s][i] = frag<C>(st, 32 * M * wm + 32 * i, s, lane);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) b[s][j] = frag<C>(st + C::ABYTES, brow[j], s, lane);
-  }
+// Byte offset of the fragment chunk of k-step s (see frag) within the 32 LDS
+// rows it starts at: the swizzle repeats every 32 rows, so fragments 32 rows
+// apart are a constant apart.
+template <class C>
+__device__ __forceinline__ int frag_off(int lane, int s) {
+  static_assert((32 / C::RPB) % C::CPR == 0, "swizzle period");
+  return swz<C>(lane & 31, 2 * s + (lane >> 5));
 }
 
-// The MFMAs of one staged step from registers, in compute_step's order.
-template <class C, int M, int DT>
-__device__ __forceinline__ void mfma_step(const u32x4_t (&a)[C::PBK / 16][M],
-                                          const u32x4_t (&b)[C::PBK / 16][2],
-                                          f32x16_t (&acc)[M][2]) {
-#pragma unroll
-  for (int s = 0; s < C::PBK / 16; ++s)
-#pragma unroll
-    for (int i = 0; i < M; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = pmfma<DT>(a[s][i], b[s][j], acc[i][j]);
-}
-
-// Ping-pong K loop (8 waves).  Waves 0-3 (half 0, one per SIMD) and waves
-// 4-7 (half 1) alternate between a memory phase (issue the loads of a future
-// step, read all fragments of the current step into registers) and an MFMA
-// phase, half a step apart, so on every SIMD one wave's MFMAs run while the
-// other wave reads its fragments; in the plain loop both waves of a SIMD
-// leave each step's barrier together and wait for their first fragments
-// together.  Barriers b(0), b(1), ... separate the phases:
-//   half 0, step k:  b(2k)  [memory k]  b(2k+1)  [MFMA k, wait loads of k+1]
-//   half 1, step k:  b(2k+1) [memory k, wait loads of k+1]  b(2k+2)  [MFMA k]
-// Step k's loads are complete in every thread before b(2k), so both halves
-// read it after that barrier; both have read step k-1 before b(2k), so the
-// loads of step k+NS-1 go into its stage after it.  Each half issues every
-// step's loads once, so the wait counts are those of k_loop; half 1 starts
-// with two barriers and half 0 ends with two, so both pass the same number.
-// Same MFMAs in the same order per output as k_loop.  (A workgroup's waves
-// go to the CU's four SIMDs in turn, so waves w and w + 4 share a SIMD; the
-// ordering argument above holds for any placement, only the overlap needs
-// it.)
+// K loop of the 256-row tile: four waves, one per SIMD, each owning 128 x 128
+// outputs (M x 4 accumulator tiles, 16 M registers each, in AGPRs).  With one
+// wave per SIMD nothing else hides a wait, so the loop is pipelined by hand:
+// while the MFMAs of one 16-deep k-step run, the fragments of the next one
+// are read into a second register set (the reads in the first groups of
+// MFMAs, so that the last one has arrived when they end) and operand loads go
+// out between the groups.
+// A step is four k-steps with one barrier B(k) before the last.  The five
+// buffers hold single operand tiles in the order B0 A0 B1 A1 ..: step k reads
+// buffers 2k and 2k + 1 (mod 5), step k + 1 the next two, and the fifth is
+// being loaded.
+//   s = 0, 1: MFMAs (k, s), reads (k, s + 1), B loads of step k + 2
+//   s = 2:    MFMAs (k, 2), reads (k, 3)
+//   B(k):     this wave's loads of step k + 1 done (vmcnt), its reads of step
+//             k done (lgkmcnt), all waves
+//   s = 3:    MFMAs (k, 3), reads (k + 1, 0), A loads of step k + 2
+// After B(k) every wave's loads of step k + 1 have landed, and both buffers of
+// step k are free: that of its B tile takes the A tile of step k + 2, that of its
+// A tile the B tile of step k + 3.  So the weights, most of which come from HBM,
+// have more than a step and a half to arrive and the rows, which other
+// workgroups of the XCD share, most of one.  A wave reads 256 fragment rows
+// per 128 x 128 outputs where two waves of 128 x 64 read 384: a third less LDS
+// traffic.
+// What bounds it: the card's power.  Under this loop the clock falls from 2.4
+// to 1.5-1.8 GHz, so time follows the energy of a flop: the operand bytes moved
+// (hence one wave per SIMD with large tiles and whole 128-byte lines per load)
+// as much as the stalls.  H = 4096, I = 14336, E = 8, same box, against the
+// 8-wave loop of two 4-wave halves half a step apart with K steps of 32 (down:
+// 128-row tiles, steps of 64) that it replaces: T = 6011 gate/up 2560 -> 2200 us
+// (1.28 PFLOP/s), down 1437 -> 1188; T = 2048 skewed 995 -> 858 and 573 -> 481;
+// T = 517, on 128-row tiles before, 430 -> 355 and 262 -> 166.  The same loop
+// with K steps of 32 in four stages took 2410 and 1340 us at T = 6011.
 template <class C, int M, int DT, bool NTB>
-__device__ __forceinline__ void k_loop_pp(const Stages& sb, const DmaLoad<C>& d, int nk,
-                                          const int (&brow)[2], f32x16_t (&acc)[M][2]) {
-  constexpr int NS = C::NSTAGE;
-  constexpr int S = C::PBK / 16;
-  constexpr int W = (NS - 2) * C::LDS_PER_STEP;
-  uint8_t* const st[4] = {sb.s0, sb.s1, sb.s2, sb.s3};
-  const bool half1 = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8)) != 0;
+struct PipeLoop {
+  static constexpr int NJ = C::NJ, AL = C::ALD, BL = C::BLD;
+  static constexpr int RG = M > 1 ? M - 1 : 1;         // MFMA groups (of NJ) that carry reads
+  static constexpr int RPG = (M + NJ + RG - 1) / RG;   // reads per such group
+  static constexpr int APG = (AL + M - 1) / M;         // A loads per group of s = 3
+  static constexpr int BPG = (BL / 2 + M - 1) / M;     // B loads per group of s = 0, 1
+
+  uint8_t* buf[5];
+  int fo[4];                // frag_off of the four k-steps
+  int arow, brow[C::NJ];    // LDS byte offsets of the wave's first row fragment, its columns
+  u32x4_t a[2][M], b[2][C::NJ];
+
+  // fragment q of k-step s: the NJ weight fragments, then the M row fragments
+  __device__ __forceinline__ void read(int set, const uint8_t* at, const uint8_t* bt, int s,
+                                       int q) {
+    if (q < NJ)
+      b[set][q] = *reinterpret_cast<const u32x4_t*>(bt + brow[q] + fo[s]);
+    else
+      a[set][q - NJ] =
+          *reinterpret_cast<const u32x4_t*>(at + arow + (q - NJ) * 32 * C::PROW + fo[s]);
+  }
+
+  // Step k, whose tiles are in buffers U = 2k and U + 1 (mod 5).
+  template <int U>
+  __device__ __forceinline__ void step(const DmaLoad<C>& d, int k, int nk,
+                                       f32x16_t (&acc)[M][C::NJ]) {
+    uint8_t* const bt = buf[U % 5];
+    uint8_t* const at = buf[(U + 1) % 5];
+    uint8_t* const bn = buf[(U + 2) % 5];
+    uint8_t* const an = buf[(U + 3) % 5];
+    uint8_t* const bnn = buf[(U + 4) % 5];
 #pragma unroll
-  for (int u = 0; u < NS - 1; ++u) dma_step<C, NTB>(d, st[u], u, nk);
-  wait_vm<W>();
-  u32x4_t a[S][M], b[S][2];
-  if (!half1) {
-    for (int k = 0; k < nk; k += NS) {
+    for (int s = 0; s < 4; ++s) {
 #pragma unroll
-      for (int u = 0; u < NS; ++u) {
-        if (u == 0 || k + u < nk) {
-          pp_barrier();                                                  // b(2k)
-          dma_step<C, NTB>(d, st[(u + NS - 1) % NS], k + u + NS - 1, nk);
-          read_step<C, M>(st[u], brow, a, b);
-          pp_barrier();                                                  // b(2k+1)
-          mfma_step<C, M, DT>(a, b, acc);
-          wait_vm<W>();
+      for (int g = 0; g < M; ++g) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = g * RPG; q < (g + 1) * RPG && q < M + NJ; ++q) {
+          if (s < 3)
+            read((s + 1) & 1, at, bt, s + 1, q);
+          else
+            read(0, an, bn, 0, q);
         }
+        if (s < 2) {
+#pragma unroll
+          for (int i = g * BPG; i < (g + 1) * BPG && i < BL / 2; ++i)
+            dma_b<C, NTB>(d, bnn, s * (BL / 2) + i, k + 2, nk);
+        } else if (s == 3) {
+#pragma unroll
+          for (int i = g * APG; i < (g + 1) * APG && i < AL; ++i) dma_a<C>(d, bt, i, k + 2, nk);
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[g][j] = pmfma<DT>(a[s & 1][g], b[s & 1][j], acc[g][j]);
       }
-    }
-    pp_barrier();
-    pp_barrier();
-  } else {
-    pp_barrier();
-    pp_barrier();
-    for (int k = 0; k < nk; k += NS) {
-#pragma unroll
-      for (int u = 0; u < NS; ++u) {
-        if (u == 0 || k + u < nk) {
-          dma_step<C, NTB>(d, st[(u + NS - 1) % NS], k + u + NS - 1, nk);
-          read_step<C, M>(st[u], brow, a, b);
-          wait_vm<W>();
-          pp_barrier();                                                  // b(2k+2)
-          mfma_step<C, M, DT>(a, b, acc);
-          pp_barrier();                                                  // b(2k+3)
-        }
+      if (s == 2) {
+        wait_vm<BL>();
+        step_barrier();
       }
     }
   }
-  // the last loads (zeros past the end) must land before the stages are reused
-  wait_vm<0>();
-  __syncthreads();
-}
+
+  __device__ __forceinline__ void run(const Stages& sb, const DmaLoad<C>& d, int nk,
+                                      const int (&first_row)[C::NJ], f32x16_t (&acc)[M][C::NJ]) {
+    const int lane = threadIdx.x & 63;
+    const int wm = (threadIdx.x >> 6) & 1;
+    buf[0] = sb.s0;
+    buf[1] = sb.s1;
+    buf[2] = sb.s2;
+    buf[3] = sb.s3;
+    buf[4] = sb.s4;
+    arow = 32 * M * wm * C::PROW;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) brow[j] = first_row[j] * C::PROW;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) fo[s] = frag_off<C>(lane, s);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+      for (int i = 0; i < BL; ++i) dma_b<C, NTB>(d, buf[2 * u], i, u, nk);
+#pragma unroll
+      for (int i = 0; i < AL; ++i) dma_a<C>(d, buf[2 * u + 1], i, u, nk);
+    }
+    wait_vm<AL + BL>();
+    step_barrier();
+#pragma unroll
+    for (int q = 0; q < NJ + M; ++q) read(0, buf[1], buf[0], 0, q);
+    int k = 0;
+    for (; k + 5 <= nk; k += 5) {
+      step<0>(d, k, nk, acc);
+      step<2>(d, k + 1, nk, acc);
+      step<4>(d, k + 2, nk, acc);
+      step<6>(d, k + 3, nk, acc);
+      step<8>(d, k + 4, nk, acc);
+    }
+    // the last nk % 5 steps in straight-line code: a branch inside the rotation
+    // would make the compiler wait for every load at each merge
+    if (k < nk) {
+      step<0>(d, k, nk, acc);
+      if (k + 1 < nk) {
+        step<2>(d, k + 1, nk, acc);
+        if (k + 2 < nk) {
+          step<4>(d, k + 2, nk, acc);
+          if (k + 3 < nk) step<6>(d, k + 3, nk, acc);
+        }
+      }
+    }
+    // the last loads (zeros past the end) must land before the buffers are reused
+    wait_vm<0>();
+    __syncthreads();
+  }
+};
 
 // The K loop shared by both GEMMs over nk steps.  At the top of step k, steps
 // k .. k+NS-2 are in flight; the thread waits for its loads of step k, the
@@ -528,27 +589,28 @@ __device__ __forceinline__ void k_loop_pp(const Stages& sb, const DmaLoad<C>& d,
 // outstanding loads: the loads of the next steps stay in flight.
 template <class C, int M, int DT, bool NTB>
 __device__ __forceinline__ void k_loop(const Stages& sb, const DmaLoad<C>& d, int nk,
-                                       const int (&brow)[2], f32x16_t (&acc)[M][2]) {
-  if constexpr (C::PP) {
-    k_loop_pp<C, M, DT, NTB>(sb, d, nk, brow, acc);
-    return;
-  }
-  constexpr int NS = C::NSTAGE;
-  uint8_t* const st[4] = {sb.s0, sb.s1, sb.s2, sb.s3};
+                                       const int (&brow)[C::NJ], f32x16_t (&acc)[M][C::NJ]) {
+  if constexpr (C::PIPE) {
+    PipeLoop<C, M, DT, NTB> loop;
+    loop.run(sb, d, nk, brow, acc);
+  } else {
+    constexpr int NS = C::NSTAGE;
+    uint8_t* const st[3] = {sb.s0, sb.s1, sb.s2};
 #pragma unroll
-  for (int u = 0; u < NS - 1; ++u) dma_step<C, NTB>(d, st[u], u, nk);
-  for (int k = 0; k < nk; k += NS) {
+    for (int u = 0; u < NS - 1; ++u) dma_step<C, NTB>(d, st[u], u, nk);
+    for (int k = 0; k < nk; k += NS) {
 #pragma unroll
-    for (int u = 0; u < NS; ++u) {
-      wait_vm<(NS - 2) * C::LDS_PER_STEP>();
-      tm_lds_barrier();
-      dma_step<C, NTB>(d, st[(u + NS - 1) % NS], k + u + NS - 1, nk);
-      if (u == 0 || k + u < nk) compute_step<C, M, DT>(st[u], brow, acc);
+      for (int u = 0; u < NS; ++u) {
+        wait_vm<(NS - 2) * C::LDS_PER_STEP>();
+        tm_lds_barrier();
+        dma_step<C, NTB>(d, st[(u + NS - 1) % NS], k + u + NS - 1, nk);
+        if (u == 0 || k + u < nk) compute_step<C, M, DT>(st[u], brow, acc);
+      }
     }
+    // the last loads (zeros past the end) must land before the stages are reused
+    wait_vm<0>();
+    __syncthreads();
   }
-  // the last loads (zeros past the end) must land before the stages are reused
-  wait_vm<0>();
-  __syncthreads();
 }
 
 // ------------------------------------------------------------- gate/up --
@@ -561,6 +623,14 @@ __device__ __forceinline__ uint8_t* h_stage(const Stages& sb, int m) {
   return base + (m % C::HROWS) * C::HSTRIDE;
 }
 
+// silu(a) b in fp32, silu(a) = a / (1 + e^-a): the hardware exponential and
+// reciprocal (each within one unit of 2^-23 before the result is rounded to 8
+// or 11 bits); the IEEE division took ten operations per value.  a = -inf and
+// NaN give NaN, e^-a = inf gives -0, as the division did.
+__device__ __forceinline__ float swiglu(float a, float b) {
+  return (a * __builtin_amdgcn_rcpf(1.0f + __expf(-a))) * b;
+}
+
 // The MFMAs and the epilogue of one gate/up tile with M accumulator tiles
 // per wave (see compute_step): SwiGLU in registers, the bf16 tile staged in
 // LDS, then a coalesced store of its `rows` rows.
@@ -571,27 +641,34 @@ __device__ __forceinline__ void gemm1_tile(const Stages& sb, const DmaLoad<C>& d
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int wm = wave & 1, wn = wave >> 1;
-  f32x16_t acc[M][2];
+  constexpr int NJ = C::NJ, NH = NJ / 2;
+  f32x16_t acc[M][NJ];
 #pragma unroll
   for (int i = 0; i < M; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-  // accumulator column blocks: j = 0 -> w1 rows 32 wn ..; j = 1 -> the same w3 rows
-  const int brow[2] = {32 * wn, C::PBN / 2 + 32 * wn};
+  // accumulator column blocks: the first NH hold w1 rows, the others the same w3 rows
+  int brow[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+    brow[j] = (j / NH) * (C::PBN / 2) + 32 * NH * wn + 32 * (j % NH);
   k_loop<C, M, DT, NTB>(sb, d, nk, brow, acc);
 #pragma unroll
-  for (int i = 0; i < M; ++i)
+  for (int i = 0; i < M; ++i) {
+    uint8_t* const hr = h_stage<C>(sb, 32 * M * wm + 32 * i + (lane & 31));
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const float a = acc[i][0][v];
-      const float b = acc[i][1][v];
-      const float hv = (a / (1.0f + __expf(-a))) * b;
-      const int m = 32 * M * wm + 32 * i + acc_row(v, lane);
-      const int c = 32 * wn + (lane & 31);
-      *reinterpret_cast<uint16_t*>(h_stage<C>(sb, m) + c * 2) = Half16<DT>::round(hv);
-    }
+    for (int j = 0; j < NH; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float hv[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) hv[v] = swiglu(acc[i][j][4 * q + v], acc[i][NH + j][4 * q + v]);
+        const u32x2_t p = {pack16<DT>(hv[0], hv[1]), pack16<DT>(hv[2], hv[3])};
+        *reinterpret_cast<u32x2_t*>(hr + (32 * NH * wn + 32 * j + acc_col(q, lane)) * 2) = p;
+      }
+  }
   __syncthreads();
   constexpr int PPR = C::PBN / 16;  // 16-byte pieces of an h row (PBN / 2 columns)
 #pragma unroll
@@ -631,8 +708,9 @@ __device__ __forceinline__ void gemm1_job(const Stages& sb, DmaLoad<C>& d,
                                           bool single, int cb, int H, int I) {
   const int n0 = cb * (C::PBN / 2);  // first h column of the block
   const size_t ebase = (size_t)e * I * H;
-  d.rb0 = pbuf(w1 + ebase, (uint32_t)((size_t)I * H * 2));
-  d.rb1 = pbuf(w3 + ebase, (uint32_t)((size_t)I * H * 2));
+  d.pb0 = w1 + ebase;
+  d.pb1 = w3 + ebase;
+  d.nb = (uint32_t)((size_t)I * H * 2);
 #pragma unroll
   for (int i = 0; i < C::BLD; ++i) {
     const int r = dma_row<C>(i);  // first half of the loads: w1 rows; second: the same w3 rows
@@ -646,8 +724,8 @@ __device__ __forceinline__ void gemm1_job(const Stages& sb, DmaLoad<C>& d,
   // the non-temporal policy (a load-only probe streams 7.1 TB/s with it, 6.2
   // without).  With several M-tiles the other jobs of the expert find them in
   // L2, so those loads stay cached.
-  if (C::NT_WEIGHTS && single)
-    gemm1_rows<C, C::MT, DT, C::NT_WEIGHTS>(sb, d, H / C::PBK, rows, p0, n0, I, h);
+  if (single)
+    gemm1_rows<C, C::MT, DT, true>(sb, d, H / C::PBK, rows, p0, n0, I, h);
   else gemm1_rows<C, C::MT, DT, false>(sb, d, H / C::PBK, rows, p0, n0, I, h);
 }
 
@@ -658,27 +736,22 @@ tm_prefill_gemm1_kernel(const uint16_t* __restrict__ x, const uint16_t* __restri
                         const int32_t* __restrict__ sorted_slots,
                         const int32_t* __restrict__ offsets, const int32_t* __restrict__ tiles,
                         int max_tiles, int E, int H, int I, int mt_max, uint32_t x_bytes) {
-  __shared__ __attribute__((aligned(16))) uint8_t s0[C::STAGE];
-  __shared__ __attribute__((aligned(16))) uint8_t s1[C::STAGE];
-  __shared__ __attribute__((aligned(16))) uint8_t s2[C::STAGE];
-  __shared__ __attribute__((aligned(16))) uint8_t s3[C::NSTAGE > 3 ? C::STAGE : 16];
-  const Stages sb{s0, s1, s2, s3};
-  int mt, cb;
-  const int ncol = I / (C::PBN / 2);
-  if (!expert_job<C>((int)blockIdx.x, offsets, E, mt_max, ncol, &mt, &cb)) return;
-  int e, p0, rows;
-  bool single;
-  if (!find_mtile<C>(offsets, tiles, max_tiles, E, mt, &e, &p0, &rows, &single)) return;
+  TM_STAGES(C);
+  Job jb;
+  if (!expert_job<C>((int)blockIdx.x, offsets, tiles, max_tiles, E, mt_max, I / (C::PBN / 2),
+                     &jb))
+    return;
   DmaLoad<C> d;
-  d.ra = pbuf(x, x_bytes);
+  d.pa = x;
+  d.na = x_bytes;
 #pragma unroll
   for (int i = 0; i < C::ALD; ++i) {
     const int r = dma_row<C>(i);
-    d.aoff[i] = r < rows ? (uint32_t)(sorted_slots[p0 + r] >> 1) * (uint32_t)H * 2u +
-                               (uint32_t)dma_chunk<C>(r) * 16u
-                         : kOOR;
+    d.aoff[i] = r < jb.rows ? (uint32_t)(sorted_slots[jb.p0 + r] >> 1) * (uint32_t)H * 2u +
+                                  (uint32_t)dma_chunk<C>(r) * 16u
+                            : kOOR;
   }
-  gemm1_job<C, DT>(sb, d, w1, w3, h, e, p0, rows, single, cb, H, I);
+  gemm1_job<C, DT>(sb, d, w1, w3, h, jb.e, jb.p0, jb.rows, jb.single, jb.col, H, I);
 }
 
 // ------------------------------------------------ gate/up, self-routed --
@@ -889,11 +962,8 @@ __global__ void __launch_bounds__(C::NT)
 tm_prefill_gemm1_routed_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w1,
                                const uint16_t* __restrict__ w3, uint16_t* __restrict__ h,
                                tmb::BucketArgs ra, int H, int I, int mt_max, uint32_t x_bytes) {
-  __shared__ __attribute__((aligned(16))) uint8_t s0[C::STAGE];
-  __shared__ __attribute__((aligned(16))) uint8_t s1[C::STAGE];
-  __shared__ __attribute__((aligned(16))) uint8_t s2[C::STAGE];
-  __shared__ __attribute__((aligned(16))) uint8_t s3[C::NSTAGE > 3 ? C::STAGE : 16];
-  static_assert(sizeof(RvShared) <= C::STAGE, "the routing writer uses the first stage");
+  TM_STAGES(C);
+  static_assert(sizeof(RvShared) <= C::BUF, "the routing writer uses the first stage");
   const int L = (int)blockIdx.x;
   if (L < kRvLeaders) {
     if (L == 0) tmb::bucket_phases<C::NT, RvShared, true>(ra, *reinterpret_cast<RvShared*>(s0));
@@ -906,7 +976,8 @@ tm_prefill_gemm1_routed_kernel(const uint16_t* __restrict__ x, const uint16_t* _
                      &single, &cb, &mask))
     return;
   DmaLoad<C> d;
-  d.ra = pbuf(x, x_bytes);
+  d.pa = x;
+  d.na = x_bytes;
 #pragma unroll
   for (int i = 0; i < C::ALD; ++i) {
     const int r = dma_row<C>(i);
@@ -914,15 +985,15 @@ tm_prefill_gemm1_routed_kernel(const uint16_t* __restrict__ x, const uint16_t* _
                                (uint32_t)dma_chunk<C>(r) * 16u
                          : kOOR;
   }
-  const Stages sb{s0, s1, s2, s3};
   gemm1_job<C, DT>(sb, d, w1, w3, h, e, p0, rows, single, cb, H, I);
 }
 
 // ---------------------------------------------------------------- down --
 // y[s, p, n] = gates_flat[slot(p)] * sum_{k in segment s} h[p, k] w2[e, n, k]
 // for the rows p of one M-tile and 256 output columns n.  The fp32 partials
-// go straight from the accumulators: for each accumulator value, 32 lanes
-// store 128 contiguous bytes of one row.
+// go straight from the accumulators, 16 bytes per lane and store; a lane's
+// rows (one per accumulator row block) have their gates loaded before the K
+// loop.
 template <class C, int M, int DT, bool NTB>
 __device__ __forceinline__ void gemm2_tile(const Stages& sb, const DmaLoad<C>& d, int nk,
                                            int rows, int p0, int H,
@@ -931,29 +1002,56 @@ __device__ __forceinline__ void gemm2_tile(const Stages& sb, const DmaLoad<C>& d
                                            float* __restrict__ ys) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = wave & 1, wn = wave >> 1;
-  f32x16_t acc[M][2];
+  constexpr int NJ = C::NJ;
+  float gate[M];
+#pragma unroll
+  for (int i = 0; i < M; ++i) {
+    const int m = 32 * M * wm + 32 * i + (lane & 31);
+    gate[i] = gates_flat[sorted_slots[p0 + min(m, rows - 1)]];
+  }
+  f32x16_t acc[M][NJ];
 #pragma unroll
   for (int i = 0; i < M; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-  const int brow[2] = {64 * wn, 64 * wn + 32};
+  int brow[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) brow[j] = 32 * NJ * wn + 32 * j;
   k_loop<C, M, DT, NTB>(sb, d, nk, brow, acc);
 #pragma unroll
-  for (int i = 0; i < M; ++i)
+  for (int i = 0; i < M; ++i) {
+    const int m = 32 * M * wm + 32 * i + (lane & 31);
+    if (m < rows) {
+      float* const yr = ys + (size_t)(p0 + m) * H + 32 * NJ * wn;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int m = 32 * M * wm + 32 * i + acc_row(v, lane);
-      if (m < rows) {
-        const float gate = gates_flat[sorted_slots[p0 + m]];
+      for (int j = 0; j < NJ; ++j)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int c = 64 * wn + 32 * j + (lane & 31);
-          ys[(size_t)(p0 + m) * H + c] = acc[i][j][v] * gate;
+        for (int q = 0; q < 4; ++q) {
+          f32x4_t o;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) o[v] = acc[i][j][4 * q + v] * gate[i];
+          *reinterpret_cast<f32x4_t*>(yr + 32 * j + acc_col(q, lane)) = o;
         }
-      }
     }
+  }
+}
+
+// gemm2_tile with the fewest accumulator tiles that cover `rows`, as gemm1_rows.
+template <class C, int MM, int DT, bool NTB>
+__device__ __forceinline__ void gemm2_rows(const Stages& sb, const DmaLoad<C>& d, int nk,
+                                           int rows, int p0, int H,
+                                           const float* __restrict__ gates_flat,
+                                           const int32_t* __restrict__ sorted_slots,
+                                           float* __restrict__ ys) {
+  if constexpr (MM > 1) {
+    if (rows <= 64 * (MM - 1)) {
+      gemm2_rows<C, MM - 1, DT, NTB>(sb, d, nk, rows, p0, H, gates_flat, sorted_slots, ys);
+      return;
+    }
+  }
+  gemm2_tile<C, MM, DT, NTB>(sb, d, nk, rows, p0, H, gates_flat, sorted_slots, ys);
 }
 
 template <class C, int DT>
@@ -964,63 +1062,49 @@ tm_prefill_gemm2_kernel(const uint16_t* __restrict__ h, const uint16_t* __restri
                         const int32_t* __restrict__ offsets, const int32_t* __restrict__ tiles,
                         int max_tiles, int E, int R, int H, int I, int klen, int nsplit,
                         int mt_max, uint32_t h_bytes) {
-  __shared__ __attribute__((aligned(16))) uint8_t s0[C::STAGE];
-  __shared__ __attribute__((aligned(16))) uint8_t s1[C::STAGE];
-  __shared__ __attribute__((aligned(16))) uint8_t s2[C::STAGE];
-  __shared__ __attribute__((aligned(16))) uint8_t s3[C::NSTAGE > 3 ? C::STAGE : 16];
-  static_assert(C::NW == 8, "down GEMM: 8 waves, 64 output columns per column group");
-  int mt, job;  // job = (segment, column block), segment-major
+  TM_STAGES(C);
   const int ncb = H / C::PBN;
-  const int ncol = ncb * nsplit;
-  if (!expert_job<C>((int)blockIdx.x, offsets, E, mt_max, ncol, &mt, &job)) return;
+  Job jb;  // col = (segment, column block), segment-major
+  if (!expert_job<C>((int)blockIdx.x, offsets, tiles, max_tiles, E, mt_max, ncb * nsplit, &jb))
+    return;
   // Each XCD owns a contiguous range of these jobs, so segment-major puts
   // one K segment on each XCD (2 segments over 8 XCDs: 4 each) and an XCD
   // reads the h rows of its segment only, instead of all of h.
-  const int seg = job / ncb;
-  const int cb = job - seg * ncb;
-  int e, p0, rows;
-  bool single;
-  if (!find_mtile<C>(offsets, tiles, max_tiles, E, mt, &e, &p0, &rows, &single)) return;
+  const int seg = jb.col / ncb;
+  const int cb = jb.col - seg * ncb;
   const int n0 = cb * C::PBN;
   const uint32_t k0 = (uint32_t)seg * (uint32_t)klen * 2u;  // segment start, bytes
 
   DmaLoad<C> d;
-  d.ra = pbuf(h, h_bytes);
-  d.rb0 = d.rb1 = pbuf(w2 + (size_t)e * H * I, (uint32_t)((size_t)H * I * 2));
+  d.pa = h;
+  d.na = h_bytes;
+  d.pb0 = d.pb1 = w2 + (size_t)jb.e * H * I;
+  d.nb = (uint32_t)((size_t)H * I * 2);
 #pragma unroll
   for (int i = 0; i < C::ALD; ++i) {
     const int r = dma_row<C>(i);
-    d.aoff[i] = r < rows ? (uint32_t)(p0 + r) * (uint32_t)I * 2u + k0 +
-                               (uint32_t)dma_chunk<C>(r) * 16u
-                         : kOOR;
+    d.aoff[i] = r < jb.rows ? (uint32_t)(jb.p0 + r) * (uint32_t)I * 2u + k0 +
+                                  (uint32_t)dma_chunk<C>(r) * 16u
+                            : kOOR;
   }
 #pragma unroll
   for (int i = 0; i < C::BLD; ++i) {
     const int r = dma_row<C>(i);
     d.boff[i] = (uint32_t)(n0 + r) * (uint32_t)I * 2u + k0 + (uint32_t)dma_chunk<C>(r) * 16u;
   }
-  const Stages sb{s0, s1, s2, s3};
   float* ys = y + (size_t)seg * R * H + n0;
-  if constexpr (C::MT > 1) {
-    if (rows <= C::PBM / 2) {  // as in gate/up
-      if (C::NT_WEIGHTS && single)
-        gemm2_tile<C, C::MT / 2, DT, C::NT_WEIGHTS>(sb, d, klen / C::PBK, rows, p0, H, gates_flat,
-                                           sorted_slots, ys);
-      else
-        gemm2_tile<C, C::MT / 2, DT, false>(sb, d, klen / C::PBK, rows, p0, H, gates_flat,
+  const int nk = klen / C::PBK;
+  if (jb.single)
+    gemm2_rows<C, C::MT, DT, true>(sb, d, nk, jb.rows, jb.p0, H, gates_flat,
                                             sorted_slots, ys);
-      return;
-    }
-  }
-  if (C::NT_WEIGHTS && single)
-    gemm2_tile<C, C::MT, DT, C::NT_WEIGHTS>(sb, d, klen / C::PBK, rows, p0, H, gates_flat, sorted_slots,
-                                   ys);
   else
-    gemm2_tile<C, C::MT, DT, false>(sb, d, klen / C::PBK, rows, p0, H, gates_flat, sorted_slots,
-                                    ys);
+    gemm2_rows<C, C::MT, DT, false>(sb, d, nk, jb.rows, jb.p0, H, gates_flat, sorted_slots, ys);
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p % 16) == 0; }
+
+// The experts average 112 rows or more: Tile256 (see tm_op1_prefill_gemm1).
+bool many_rows(int64_t T, int64_t E) { return 2 * T >= 112 * E; }
 
 // The gate/up launch with tile C: jobs for the M-tile bound (the tile list's
 // length, capped by what 2T rows in E experts can take).
@@ -1075,14 +1159,17 @@ extern "C" int tm_op1_prefill_gemm1(const void* x, const void* w1, const void* w
   if (I * H * 2 >= (int64_t)kOOR || T * H * 2 >= (int64_t)kOOR || 2 * T * I * 2 >= (int64_t)kOOR)
     return TM_ERR_SHAPE;
   if (!aligned16(x) || !aligned16(w1) || !aligned16(w3) || !aligned16(h)) return TM_ERR_ALIGN;
-  // 256-row tiles when the experts average 384 rows or more: they read fewer
-  // operand bytes per flop, but below that their coarser jobs and padding
-  // cost more than that saves (measured at the Mixtral shape).  TileDec when
+  // 256-row tiles where the experts average 112 rows or more: from there an
+  // expert often has more rows than a 128-row tile holds, and its weights would
+  // pass through LDS twice.  H = 4096, I = 14336, E = 8, gate/up + down on
+  // Tile128 against Tile256: T = 400 490 against 502 us, T = 430 496 against
+  // 503, T = 460 (115 rows) 580 against 505, T = 517 680 against 519, T = 1030
+  // 918 against 896.  TileDec when
   // the tile list leaves at most 16 rows per entry (2T <= 16 max_tiles: few
   // rows per active expert, e.g. 64 tree tokens over 8 experts): half the
   // weight rows per workgroup and two workgroups per CU stream the weights
   // faster there (config 2 gate/up 302 -> 289 us same-box).
-  const bool big = 2 * T >= 384 * E;
+  const bool big = many_rows(T, E);
   const bool dec = !big && 2 * T <= 16 * max_tiles;
   const hipStream_t st = (hipStream_t)stream;
   const bool f16 = dtype == TM_DTYPE_F16;
@@ -1148,8 +1235,8 @@ extern "C" int tm_op1_prefill_gemm1_routed(
   ra.sorted_slots = sorted_slots;
   ra.slot_pos = slot_pos;
   ra.tiles = tiles;
-  // the tile rule of tm_op1_prefill_gemm1 (2T < 384 E here, so never the
-  // 256-row tile)
+  // the tile rule of tm_op1_prefill_gemm1 without the 256-row tile (T <= 64: at
+  // most 64 rows per expert)
   const bool dec = 2 * T <= 16 * max_tiles;
   const hipStream_t st = (hipStream_t)stream;
   const bool f16 = dtype == TM_DTYPE_F16;
@@ -1203,10 +1290,8 @@ extern "C" int tm_op1_prefill_gemm2(const void* h, const void* w2, float* y,
   if (klen < C::PBK || (klen % C::PBK) != 0 || H < C::PBN || (H % C::PBN) != 0) return TM_ERR_SHAPE;
   if (H * I * 2 >= (int64_t)kOOR || 2 * T * I * 2 >= (int64_t)kOOR) return TM_ERR_SHAPE;
   if (!aligned16(h) || !aligned16(w2) || !aligned16(y)) return TM_ERR_ALIGN;
-  // where the experts average 384 rows or more (the gate/up rule for its
-  // 256-row tile) the MFMAs bound the kernel and the ping-pong loop runs
-  const bool big = 2 * T >= 384 * E;
-  const int rc = big ? launch_gemm2<Tile128PP>(h, w2, y, gates_flat, sorted_slots,
+  const bool big = many_rows(T, E);  // the gate/up rule
+  const int rc = big ? launch_gemm2<Tile256>(h, w2, y, gates_flat, sorted_slots,
                                                expert_offsets, tiles, max_tiles, split, T, H,
                                                I, E, dtype, (hipStream_t)stream)
                      : launch_gemm2<Tile128>(h, w2, y, gates_flat, sorted_slots, expert_offsets,

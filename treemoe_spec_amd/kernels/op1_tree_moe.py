@@ -82,10 +82,12 @@ def uses_tiled_gemms(num_tokens: int, expert_budget: int, num_experts: int,
 
 def tiled_gate_up_tile(num_tokens: int, num_experts: int, max_tiles: int) -> str:
     """The tile tm_op1_prefill_gemm1 picks (the rule in op1_prefill.hip):
-    256-row tiles when the experts average 384 rows or more, the 64-row
+    256-row tiles when the experts average 112 rows or more, the 64-row
     decode tile when the tile list leaves at most 16 rows per entry, else
-    128-row tiles.  For naming kernels in measurements."""
-    if 2 * num_tokens >= 384 * num_experts:
+    128-row tiles.  For naming kernels in measurements: the labels stay the same
+    from build to build, so the 256-row tile keeps the one it had with K steps
+    of 32 and four stages."""
+    if 2 * num_tokens >= 112 * num_experts:
         return "Tile<256, 32, 4>"
     if 2 * num_tokens <= 16 * max_tiles:
         return "Tile<64, 64, 3, 128, 256>"
