@@ -341,6 +341,10 @@ __global__ void __launch_bounds__(kThreads, 2) tm_tree_attn_kernel(AttnParams p)
 
   // this lane's query (column c32 of the wave's 32): Q^T fragments, mask row
   const int row = rb * kRows + wave * 32 + c32;
+  // a wave whose 32 rows all lie past the last one (one token has `group` rows)
+  // only helps to stage the keys; its LDS reads and MFMAs would slow the others
+  const bool wave_rows =
+      __builtin_amdgcn_readfirstlane(rb * kRows + (tid >> 6) * 32) < p.rows;
   const bool row_ok = row < p.rows;
   const int node = row_ok ? row % p.n : 0;
   const int head = kvhead * p.group + (row_ok ? row / p.n : 0);
@@ -383,7 +387,8 @@ __global__ void __launch_bounds__(kThreads, 2) tm_tree_attn_kernel(AttnParams p)
     const int kb = c0 + s * kKeys, kn = kb + kKeys;
     const bool more = s + 1 < nstage;
     if (more) load_stage(p, s_pages, kn, c0, c1, head_off, quad, st);
-    attend_stage(p, s_buf + (s & 1) * kStage, kb, c1, mw, half, c32, qf, acc, m_run, l_run);
+    if (wave_rows)
+      attend_stage(p, s_buf + (s & 1) * kStage, kb, c1, mw, half, c32, qf, acc, m_run, l_run);
     if (more) {
       if (write_rows && kn + kKeys > p.seq_len)
         store_tree_rows(p, s_tpages, kn, c1, quad, head_off, st);
@@ -392,6 +397,7 @@ __global__ void __launch_bounds__(kThreads, 2) tm_tree_attn_kernel(AttnParams p)
     }
   }
 
+  if (!wave_rows) return;
   // the two lanes of a query hold partial sums over disjoint keys
   l_run += __shfl_xor(l_run, 32);
   const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
@@ -434,25 +440,30 @@ __global__ void __launch_bounds__(kThreads, 2) tm_tree_attn_kernel(AttnParams p)
   }
 }
 
-// One thread per (KV head, row block, wave, 4-value group, lane): merges the
-// chunks' normalised partials in chunk order with a running maximum,
+// One workgroup per (KV head, row block, 32-row group, 4-value group): its four
+// waves merge the chunks c with c % 4 = wave, in chunk order with a running
+// maximum,
 //   w_c = l_c 2^(m_c - M),  O = sum_c w_c O_c / sum_c w_c,
-// keeping the running sums against the running maximum.  Branch-free, so the
-// loads of later chunks can issue early.
+// keeping the running sums against the running maximum, and the first wave
+// merges the four in wave order.  The kernel is bound by the latency of its
+// loads: one wave over all chunks waited for four at a time, one after the
+// other.  Whole call, 32 query over 8 KV heads, together with the waves without
+// rows above: one node over 1000 / 3000 / 7777 positions 11.9 / 16.0 / 19.0 ->
+// 9.5 / 11.8 / 15.3 us, 27 nodes over 333 11.5 -> 10.5, 64 over 4096 20.0 -> 20.0.
 __global__ void __launch_bounds__(kThreads) tm_tree_attn_combine_kernel(AttnParams p) {
-  const int64_t u = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  const int lane = (int)(u & 63);
-  const int grp = (int)((u >> 6) & 15);       // (ht, gq) = (grp / 4, grp % 4)
-  const int64_t kw = u >> 10;                 // (kvhead * row_blocks + rb) * 4 + wave
-  const int wave = (int)(kw & 3);
-  const int64_t kr = kw >> 2;
-  if (kr >= (int64_t)p.kvh * p.row_blocks) return;
+  __shared__ float s_o[3][6][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int grp = (int)(blockIdx.x & 15);     // (ht, gq) = (grp / 4, grp % 4)
+  const int kw = (int)(blockIdx.x >> 4);      // (kvhead * row_blocks + rb) * 4 + 32-row group
+  const int rg = kw & 3, kr = kw >> 2;
+  const int rb = kr % p.row_blocks, kvhead = kr / p.row_blocks;
+  if (rb * kRows + rg * 32 >= p.rows) return;
   const int c32 = lane & 31, half = lane >> 5;
   float m_run = -INFINITY, w_sum = 0.0f;
   f32x4_t o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
-  for (int c = 0; c < p.chunks; ++c) {
-    const int64_t slot = (kr * p.chunks + c) * 4 + wave;
+  for (int c = wave; c < p.chunks; c += 4) {
+    const int64_t slot = ((int64_t)kr * p.chunks + c) * 4 + rg;
     const f32x2_t st = *reinterpret_cast<const f32x2_t*>(p.stats + slot * kStatFloats + c32 * 2);
     const f16x4_t hc = *reinterpret_cast<const f16x4_t*>(
         reinterpret_cast<const _Float16*>(p.part) + slot * kPartHalves + grp * 256 + lane * 4);
@@ -467,10 +478,26 @@ __global__ void __launch_bounds__(kThreads) tm_tree_attn_combine_kernel(AttnPara
     o[3] = o[3] * a + (float)hc[3] * b;
     m_run = mn;
   }
-  const int rb = (int)(kr % p.row_blocks);
-  const int kvhead = (int)(kr / p.row_blocks);
-  const int row = rb * kRows + wave * 32 + c32;
-  if (row >= p.rows) return;
+  if (wave > 0) {
+    s_o[wave - 1][0][lane] = m_run;
+    s_o[wave - 1][1][lane] = w_sum;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) s_o[wave - 1][2 + v][lane] = o[v];
+  }
+  __syncthreads();
+  const int row = rb * kRows + rg * 32 + c32;
+  if (wave > 0 || row >= p.rows) return;
+#pragma unroll
+  for (int w = 0; w < 3; ++w) {
+    const float m2 = s_o[w][0][lane];
+    const float mn = fmaxf(m_run, m2);
+    const float ref = mn == -INFINITY ? 0.0f : mn;
+    const float a = exp2f(m_run - ref), b = exp2f(m2 - ref);
+    w_sum = w_sum * a + s_o[w][1][lane] * b;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) o[v] = o[v] * a + s_o[w][2 + v][lane] * b;
+    m_run = mn;
+  }
   const int node = row % p.n;
   const int head = kvhead * p.group + row / p.n;
   const float inv = w_sum > 0.0f ? 1.0f / w_sum : 0.0f;
@@ -535,17 +562,17 @@ int64_t groups_of(int64_t kvh, int64_t row_blocks, int64_t chunks) {
 // Planner cost of a split, in units of one 64-key stage of one workgroup:
 // the longest chunk's stages plus ~2 stages of workgroup prologue and
 // epilogue, times 1.6 per extra workgroup a CU has to hold (co-resident
-// workgroups share its SIMDs), plus, with several chunks, ~2 stages for the
-// combine kernel's launch and 0.1 per chunk it merges (its loop over the
-// chunks).  Fitted to measurements on MI355X at 1024 .. 16384 cached positions
-// (N = 64, 32 query and 8 KV heads), where it picks the fastest chunk length
-// of those tried.
+// workgroups share its SIMDs), plus, with several chunks, ~1.6 stages for the
+// combine kernel's launch and 0.04 per chunk it merges (four waves share its
+// loop over the chunks).  Fitted to measurements on MI355X at 1 .. 64 nodes and
+// 40 .. 8000 cached positions (32 query heads over 8 KV heads, 8 over 2), where
+// it picks the fastest chunk length of those tried or one within 4 % of it.
 double split_cost(const Split& sp, int64_t s_total, int64_t kvh, int64_t row_blocks) {
   const int64_t keys = sp.chunks > 1 ? sp.len : s_total;
   const double stages = (double)((keys + kKeys - 1) / kKeys);
   const int64_t groups = groups_of(kvh, row_blocks, sp.chunks);
   const double stretch = groups <= kCUs ? 1.0 : 0.8 * (double)((groups + kCUs - 1) / kCUs);
-  const double combine = sp.chunks > 1 ? 2.0 + 0.1 * (double)sp.chunks : 0.0;
+  const double combine = sp.chunks > 1 ? 1.6 + 0.04 * (double)sp.chunks : 0.0;
   return (stages + 2.0) * stretch + combine;
 }
 
@@ -700,10 +727,10 @@ extern "C" int tm_tree_attention(const void* q, int64_t q_stride, const void* k_
                      (hipStream_t)stream, p);
   TM_HIP_CHECK_LAUNCH();
   if (pl.chunks > 1) {
-    // kvh * row_blocks * 4 waves * 16 groups * 64 lanes threads
+    // KV heads x row blocks x four 32-row groups x 16 value groups
     hipLaunchKernelGGL(tm_tree_attn_combine_kernel,
-                       dim3((unsigned)(kvh * pl.row_blocks * 4 * 16 * 64 / kThreads)),
-                       dim3(kThreads), 0, (hipStream_t)stream, p);
+                       dim3((unsigned)(kvh * pl.row_blocks * 4 * 16)), dim3(kThreads), 0,
+                       (hipStream_t)stream, p);
     TM_HIP_CHECK_LAUNCH();
   }
   return TM_OK;
