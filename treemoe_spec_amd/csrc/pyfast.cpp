@@ -1,5 +1,5 @@
-// _tmfast: a CPython binding of the per-step op4 greedy path of
-// libtreemoe_amd.so.  The ctypes binding converts each argument through a
+// _tmfast: a CPython binding of the per-step op4 greedy path and of the
+// per-layer tree attention of libtreemoe_amd.so.  The ctypes binding converts each argument through a
 // Python-level type object (~3.5 us per call of ~18 arguments on the GPU
 // host); this module parses them with PyArg_ParseTuple and calls the C ABI
 // directly, so one greedy verify + KV commit costs one Python-to-C
@@ -52,7 +52,38 @@ PyObject* py_kv_commit(PyObject*, PyObject* args) {
   return PyLong_FromLong(rc);
 }
 
+// attn_workspace(N, Hq, kvh, hd, seq_len, page_size, chunk_keys)
+//   -> (status, workspace bytes)
+PyObject* py_attn_workspace(PyObject*, PyObject* args) {
+  long long n, hq, kvh, hd, seq, page, chunk;
+  if (!PyArg_ParseTuple(args, "LLLLLLL", &n, &hq, &kvh, &hd, &seq, &page, &chunk)) return nullptr;
+  int64_t chunks = 0, bytes = 0;
+  const int rc = tm_tree_attention_plan(n, hq, kvh, hd, seq, page, chunk, &chunks, &bytes);
+  return Py_BuildValue("iL", rc, (long long)bytes);
+}
+
+// tree_attention(...) -> status, the arguments of tm_tree_attention in order
+PyObject* py_tree_attention(PyObject*, PyObject* args) {
+  unsigned long long q, kt, vt, kc, vc, table, scratch, mask, out, ws, stream;
+  long long qs, ts, sp, ss, page, n_table, seq, n_scratch, n, hq, kvh, hd, os, chunk, ws_bytes;
+  int write_tree;
+  float scale;
+  if (!PyArg_ParseTuple(args, "KLKKLKKLLLKLLKLiKLLLLfKLLKLK", &q, &qs, &kt, &vt, &ts, &kc, &vc,
+                        &sp, &ss, &page, &table, &n_table, &seq, &scratch, &n_scratch,
+                        &write_tree, &mask, &n, &hq, &kvh, &hd, &scale, &out, &os, &chunk, &ws,
+                        &ws_bytes, &stream))
+    return nullptr;
+  const int rc = tm_tree_attention(
+      (const void*)q, qs, (const void*)kt, (const void*)vt, ts, (void*)kc, (void*)vc, sp, ss, page,
+      (const int32_t*)table, n_table, seq, (const int32_t*)scratch, n_scratch, write_tree,
+      (const uint64_t*)mask, n, hq, kvh, hd, scale, (void*)out, os, chunk, (void*)ws, ws_bytes,
+      (void*)stream);
+  return PyLong_FromLong(rc);
+}
+
 PyMethodDef kMethods[] = {
+    {"attn_workspace", py_attn_workspace, METH_VARARGS, "tm_tree_attention_plan"},
+    {"tree_attention", py_tree_attention, METH_VARARGS, "tm_tree_attention"},
     {"argmax_walk", py_argmax_walk, METH_VARARGS, "tm_op4_argmax_walk"},
     {"kv_commit", py_kv_commit, METH_VARARGS, "tm_op4_kv_commit"},
     {nullptr, nullptr, 0, nullptr},

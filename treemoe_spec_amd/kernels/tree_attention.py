@@ -18,13 +18,24 @@ stored into the scratch pages by the same kernel.  The context comes back as
 from __future__ import annotations
 
 import ctypes
+import operator
 import weakref
 
 import torch
 
 from treemoe_spec_amd import _capi
-from treemoe_spec_amd._capi import call, ptr
+from treemoe_spec_amd._capi import call, check, ptr
 from treemoe_spec_amd.kv_cache import device_tables_of, scratch_pages_of
+
+# Called once per layer of every forward: the C ABI goes through the CPython
+# binding where it is built, and a layer's cache is addressed by its offset
+# instead of through a tensor view.  Host time of a call 14-17 -> 8 us, which
+# is what bounded the short contexts (27 nodes over 333 positions: 10.5 us on
+# the device).
+try:
+    from treemoe_spec_amd import _tmfast as _fast
+except ImportError:  # not built: the ctypes binding is used
+    _fast = None
 
 _mask_cache: dict = {}
 
@@ -61,20 +72,29 @@ def tree_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv, layer:
         raise RuntimeError("treemoe_spec_amd tree attention runs on ROCm devices only; "
                            "got a CPU tensor")
     n, hq, hd = q.shape
-    if k.shape[0] != n or v.shape != k.shape or k.dim() != 3:
+    kshape = k.shape
+    if kshape[0] != n or v.shape != kshape or len(kshape) != 3:
         raise ValueError("k and v must be [N, kv_heads, head_dim] like q's N")
-    kvh = k.shape[1]
+    kvh = kshape[1]
     if hq % kvh != 0:
         raise ValueError("num_heads must be a multiple of num_kv_heads")
-    for name, t in (("q", q), ("k", k), ("v", v)):
+    qs, ks, vs = q.stride(), k.stride(), v.stride()
+    for name, t, st in (("q", q, qs), ("k", k, ks), ("v", v, vs)):
         if t.dtype != torch.bfloat16:
             raise ValueError(f"{name} must be bfloat16")
-        if t.stride(2) != 1 or t.stride(1) != hd:
+        if st[2] != 1 or st[1] != hd:
             raise ValueError(f"{name} must have contiguous heads")
-    if k.stride(0) != v.stride(0):
+    if ks[0] != vs[0]:
         raise ValueError("k and v must share the node stride")
-    if kv.k.dtype != torch.bfloat16 or kv.k.shape[3] != kvh or kv.k.shape[4] != hd:
+    kc, vc = kv.k, kv.v
+    cshape = kc.shape
+    if kc.dtype != torch.bfloat16 or cshape[3] != kvh or cshape[4] != hd:
         raise ValueError("cache layout must be [L, pages, page, kv_heads, head_dim] bf16")
+    layer = operator.index(layer)
+    if not -cshape[0] <= layer < cshape[0]:
+        raise IndexError(f"layer {layer} is out of range for a cache of {cshape[0]} layers")
+    if layer < 0:
+        layer += cshape[0]
     if tuple(tree_mask.shape) != (n, n):
         raise ValueError("tree_mask must be [N, N]")
     dev = q.device
@@ -82,26 +102,36 @@ def tree_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv, layer:
         scale = hd ** -0.5
     bits = pack_tree_mask(tree_mask)
     pages = scratch_pages_of(kv)
-    if write_tree and len(pages) * kv.block_size < n:
+    page = kv.block_size
+    if write_tree and len(pages) * page < n:
         raise ValueError("tree larger than the KV scratch pages")
     table, scratch = device_tables_of(kv, dev)
     seq_len = kv.seq_len
-    chunks = ctypes.c_int64()
-    wbytes = ctypes.c_int64()
-    call("tm_tree_attention_plan", n, hq, kvh, hd, seq_len, kv.block_size, chunk_keys,
-         ctypes.byref(chunks), ctypes.byref(wbytes))
-    ws = _workspace(wbytes.value, dev)
+    if _fast is not None:
+        rc, nbytes = _fast.attn_workspace(n, hq, kvh, hd, seq_len, page, chunk_keys)
+        check(rc, "tm_tree_attention_plan")
+    else:
+        chunks = ctypes.c_int64()
+        wbytes = ctypes.c_int64()
+        call("tm_tree_attention_plan", n, hq, kvh, hd, seq_len, page, chunk_keys,
+             ctypes.byref(chunks), ctypes.byref(wbytes))
+        nbytes = wbytes.value
+    ws = _workspace(nbytes, dev)
     if out is None:
         out = torch.empty(n, hq * hd, dtype=torch.bfloat16, device=dev)
     elif out.shape != (n, hq * hd) or out.dtype != torch.bfloat16 or not out.is_contiguous():
         raise ValueError("out must be a contiguous [N, Hq * hd] bf16 tensor")
-    kc = kv.k[layer]
-    vc = kv.v[layer]
-    call("tm_tree_attention", ptr(q), q.stride(0), ptr(k), ptr(v), k.stride(0), ptr(kc),
-         ptr(vc), kc.stride(0), kc.stride(1), kv.block_size, ptr(table),
-         max(1, len(kv.block_table)), seq_len, ptr(scratch), len(pages),
-         1 if write_tree else 0, ptr(bits), n, hq, kvh, hd, float(scale), ptr(out), hq * hd,
-         chunk_keys, ptr(ws), wbytes.value, _capi.stream_of(dev))
+    cs, vcs = kc.stride(), vc.stride()
+    args = (q.data_ptr(), qs[0], k.data_ptr(), v.data_ptr(), ks[0],
+            kc.data_ptr() + 2 * layer * cs[0], vc.data_ptr() + 2 * layer * vcs[0], cs[1], cs[2],
+            page, table.data_ptr(), max(1, len(kv.block_table)), seq_len, scratch.data_ptr(),
+            len(pages), 1 if write_tree else 0, bits.data_ptr(), n, hq, kvh, hd, float(scale),
+            out.data_ptr(), hq * hd, chunk_keys, 0 if ws is None else ws.data_ptr(), nbytes,
+            _capi.stream_of(dev))
+    if _fast is not None:
+        check(_fast.tree_attention(*args), "tm_tree_attention")
+    else:
+        call("tm_tree_attention", *args)
     return out
 
 
