@@ -339,4 +339,191 @@ __device__ void bucket_phases(const BucketArgs& a, SH& sh) {
   }
 }
 
+// The kept experts (bit e) from the demand and criticality of every token
+// held in its lane (T <= 64; g: the lane's gates, zero past E or T; a_ld: the
+// lane's accept probability, loaded with the gates), as the phases compute
+// them; acc[e] becomes expert e's demand.
+template <int EM>
+__device__ __forceinline__ unsigned long long keep_set(const BucketArgs& a,
+                                                       const float (&g)[EM], float a_ld,
+                                                       bool tok, int lane, float (&acc)[EM]) {
+  const int E = a.E;
+  const float av = tok ? a_ld : 0.0f;
+  const bool critical = a.objective == TM_OBJECTIVE_CRITICAL_PATH;
+  // demand: the EM halving trees, level by level
+#pragma unroll
+  for (int e = 0; e < EM; ++e) {
+    float z = 0.0f;
+    const float p = av * g[e];
+    acc[e] = tok ? z + p : z;
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1)
+#pragma unroll
+    for (int e = 0; e < EM; ++e) acc[e] = acc[e] + __shfl_xor(acc[e], off);
+  float d_mine = 0.0f;
+#pragma unroll
+  for (int e = 0; e < EM; ++e) d_mine = lane == e ? acc[e] : d_mine;
+  float c_mine = 0.0f;
+  if (critical) {
+    Top2 u{-1, -1, 0.0f, 0.0f};
+#pragma unroll
+    for (int e = 0; e < EM; ++e)
+      if (e < E) u.offer(g[e], e);
+    float crit[EM];
+#pragma unroll
+    for (int e = 0; e < EM; ++e) {
+      const bool needed = tok && ((u.i1 == e) || ((u.i2 == e) && (av >= a.tau)));
+      crit[e] = needed ? fmaxf(-INFINITY, av) : -INFINITY;
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1)
+#pragma unroll
+      for (int e = 0; e < EM; ++e) crit[e] = fmaxf(crit[e], __shfl_xor(crit[e], off));
+#pragma unroll
+    for (int e = 0; e < EM; ++e) c_mine = lane == e ? crit[e] : c_mine;
+  }
+  // keep set: lane = expert, as in the phases
+  {
+    const float d = lane < E ? d_mine : 0.0f;
+    const float c = (critical && lane < E) ? c_mine : 0.0f;
+    int rank = 0;
+#pragma unroll
+    for (int f = 0; f < EM; ++f) {
+      if (f < E) {
+        const float df = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
+                                                       __builtin_bit_cast(int, acc[f])));
+        const float cf = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c), f));
+        bool before;
+        if (critical && cf != c) {
+          before = cf > c;
+        } else if (df != d) {
+          before = df > d;
+        } else {
+          before = f < lane;
+        }
+        rank += before ? 1 : 0;
+      }
+    }
+    return __ballot(lane < E && rank < a.budget);
+  }
+}
+
+// Budget routing and bucketing of T <= 64 tokens and E <= EM experts by NT / 64
+// waves without LDS or barriers: lane t of every wave holds token t's gates g
+// (zero past E or T) and accept probability a_ld, so every wave takes the same
+// decisions with cross-lane operations, in the order of bucket_phases, and the
+// waves share the writes.  The slots of expert e in slot order are the tokens
+// whose top-2 holds e (the two picks differ), so ranks and counts are
+// popcounts of one ballot per expert.
+template <int NT, int EM>
+__device__ __forceinline__ void bucket_wave(const BucketArgs& a, const float (&g)[EM],
+                                            float a_ld) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const bool writer = tid < 64;  // the first wave writes the per-token outputs
+  const int T = a.T, E = a.E;
+  const bool tok = lane < T;
+  float demand[EM];
+  const unsigned long long keep = keep_set<EM>(a, g, a_ld, tok, lane, demand);
+  Top2 r{-1, -1, 0.0f, 0.0f};
+#pragma unroll
+  for (int e = 0; e < EM; ++e)
+    if (e < E) r.offer(((keep >> e) & 1ull) ? g[e] : 0.0f, e);
+  const int i1 = tok ? r.i1 : -1, i2 = tok ? r.i2 : -1;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  int cnt[EM], off[EM], bs[EM], ts[EM];
+  int run_off = 0, run_blk = 0, run_tile = 0;
+  int pos1 = 0, pos2 = 0, row1 = 0, row2 = 0;
+#pragma unroll
+  for (int e = 0; e < EM; ++e) {
+    const unsigned long long m = __ballot(i1 == e || i2 == e);
+    const int rank = __popcll(m & below);
+    cnt[e] = __popcll(m);
+    off[e] = run_off;
+    bs[e] = run_blk;
+    ts[e] = run_tile;
+    if (i1 == e) {
+      pos1 = run_off + rank;
+      row1 = run_blk * a.BM + rank;
+    }
+    if (i2 == e) {
+      pos2 = run_off + rank;
+      row2 = run_blk * a.BM + rank;
+    }
+    run_off += cnt[e];
+    run_blk += (cnt[e] + a.BM - 1) / a.BM;
+    run_tile += (cnt[e] + TM_GEMM_TILE_M - 1) / TM_GEMM_TILE_M;
+  }
+  const int padded_rows = a.max_blocks * a.BM;
+  if (writer && tok) {
+    const float s = r.g1 + r.g2;
+    float tg1 = r.g1 / s;
+    float tg2 = r.g2 / s;
+    if (a_ld < a.tau) {
+      tg1 = 1.0f;
+      tg2 = 0.0f;
+    }
+    a.topk_ids[2 * lane] = i1;
+    a.topk_ids[2 * lane + 1] = i2;
+    a.gates_flat[2 * lane] = tg1;
+    a.gates_flat[2 * lane + 1] = tg2;
+    a.slot_pos[2 * lane] = pos1;
+    a.slot_pos[2 * lane + 1] = pos2;
+    a.sorted_slots[pos1] = 2 * lane;
+    a.sorted_slots[pos2] = 2 * lane + 1;
+    a.slot_to_row[2 * lane] = row1;
+    a.slot_to_row[2 * lane + 1] = row2;
+    if (row1 < padded_rows) a.padded_slots[row1] = 2 * lane;
+    if (row2 < padded_rows) a.padded_slots[row2] = 2 * lane + 1;
+  }
+  if (writer && lane < E) {
+    float d = 0.0f;
+    int o = 0;
+#pragma unroll
+    for (int e = 0; e < EM; ++e)
+      if (lane == e) {
+        d = demand[e];
+        o = off[e];
+      }
+    a.demand_out[lane] = d;
+    a.expert_offsets[lane] = o;
+    if (lane == 0) a.expert_offsets[E] = run_off;
+  }
+  // the entries without a slot: padded rows past an expert's count or in unused
+  // blocks, owners of the blocks, the tile list
+  for (int i = tid; i < padded_rows; i += NT) {
+    const int b = i / a.BM;
+    bool pad = true;
+#pragma unroll
+    for (int e = 0; e < EM; ++e) {
+      const int k = i - bs[e] * a.BM;
+      if (k >= 0 && k < cnt[e]) pad = false;
+    }
+    if (pad) a.padded_slots[i] = -1;
+    if (i == b * a.BM) {
+      int owner = -1;
+#pragma unroll
+      for (int e = 0; e < EM; ++e)
+        if (b >= bs[e] && b < bs[e] + (cnt[e] + a.BM - 1) / a.BM) owner = e;
+      a.block_expert_ids[b] = owner;
+    }
+  }
+  for (int j = tid; j < a.max_tiles; j += NT) {
+    int te = -1, r0 = 0, rows = 0;
+#pragma unroll
+    for (int e = 0; e < EM; ++e) {
+      const int k = j - ts[e];
+      if (k >= 0 && k * TM_GEMM_TILE_M < cnt[e]) {
+        te = e;
+        r0 = off[e] + k * TM_GEMM_TILE_M;
+        rows = min(TM_GEMM_TILE_M, cnt[e] - k * TM_GEMM_TILE_M);
+      }
+    }
+    a.tiles[4 * j] = te;
+    a.tiles[4 * j + 1] = r0;
+    a.tiles[4 * j + 2] = rows;
+    a.tiles[4 * j + 3] = 0;
+  }
+}
+
 }  // namespace tmb

@@ -793,76 +793,6 @@ __device__ __forceinline__ int nth_set_bit(unsigned long long m, int j) {
   return pos;
 }
 
-// The kept experts (bit e) from the demand and criticality of every token
-// held in its lane (g: the lane's gates, zero past E or T; a_ld: the lane's
-// accept probability, loaded with the gates), as the phases compute them.
-template <int EM>
-__device__ __forceinline__ unsigned long long keep_set(const tmb::BucketArgs& a,
-                                                       const float (&g)[EM], float a_ld,
-                                                       bool tok, int lane) {
-  const int E = a.E;
-  const float av = tok ? a_ld : 0.0f;
-  const bool critical = a.objective == TM_OBJECTIVE_CRITICAL_PATH;
-  // demand: the EM halving trees, level by level
-  float acc[EM];
-#pragma unroll
-  for (int e = 0; e < EM; ++e) {
-    float z = 0.0f;
-    const float p = av * g[e];
-    acc[e] = tok ? z + p : z;
-  }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1)
-#pragma unroll
-    for (int e = 0; e < EM; ++e) acc[e] = acc[e] + __shfl_xor(acc[e], off);
-  float d_mine = 0.0f;
-#pragma unroll
-  for (int e = 0; e < EM; ++e) d_mine = lane == e ? acc[e] : d_mine;
-  float c_mine = 0.0f;
-  if (critical) {
-    tmb::Top2 u{-1, -1, 0.0f, 0.0f};
-#pragma unroll
-    for (int e = 0; e < EM; ++e)
-      if (e < E) u.offer(g[e], e);
-    float crit[EM];
-#pragma unroll
-    for (int e = 0; e < EM; ++e) {
-      const bool needed = tok && ((u.i1 == e) || ((u.i2 == e) && (av >= a.tau)));
-      crit[e] = needed ? fmaxf(-INFINITY, av) : -INFINITY;
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1)
-#pragma unroll
-      for (int e = 0; e < EM; ++e) crit[e] = fmaxf(crit[e], __shfl_xor(crit[e], off));
-#pragma unroll
-    for (int e = 0; e < EM; ++e) c_mine = lane == e ? crit[e] : c_mine;
-  }
-  // keep set: lane = expert, as in the phases
-  {
-    const float d = lane < E ? d_mine : 0.0f;
-    const float c = (critical && lane < E) ? c_mine : 0.0f;
-    int rank = 0;
-#pragma unroll
-    for (int f = 0; f < EM; ++f) {
-      if (f < E) {
-        const float df = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
-                                                       __builtin_bit_cast(int, acc[f])));
-        const float cf = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c), f));
-        bool before;
-        if (critical && cf != c) {
-          before = cf > c;
-        } else if (df != d) {
-          before = df > d;
-        } else {
-          before = f < lane;
-        }
-        rank += before ? 1 : 0;
-      }
-    }
-    return __ballot(lane < E && rank < a.budget);
-  }
-}
-
 // The job of GEMM launch index l (M-tile of BM rows of one expert x column
 // block, job_of over the layer's real M-tiles) from the router gates, in one
 // wave: lane t holds token t's gates, EM >= E registers of them.  The expert
@@ -911,7 +841,10 @@ __device__ __forceinline__ bool rr_job(const tmb::BucketArgs& a, int l, int ncol
   }
   // with a budget of every expert, all are kept whatever the demand
   unsigned long long keep = (1ull << E) - 1ull;
-  if (a.budget < E) keep = keep_set<EM>(a, g, a_ld, tok, lane);
+  if (a.budget < E) {
+    float demand[EM];
+    keep = tmb::keep_set<EM>(a, g, a_ld, tok, lane, demand);
+  }
   // masked top-2 of this lane's token
   tmb::Top2 r{-1, -1, 0.0f, 0.0f};
 #pragma unroll
