@@ -76,3 +76,41 @@ def test_tile256_gemms_match_float64(steps):
             ref, mag = gate * (a @ w.T), gate * (a.abs() @ w.abs().T)
             tol = (half + 2) * 2.0 ** -24 * mag
             assert torch.all((out[s, r] - ref).abs() <= tol), (steps, COUNTS[k], s)
+
+
+@pytest.mark.parametrize("counts", [[16] * 8, [1, 15, 64, 65, 3, 0, 28, 0], [2, 2], [128, 0, 0, 0]])
+def test_narrow_down_tile_matches_float64(counts):
+    """Down with too few 128-row jobs for the chip (64-row tiles, 128 columns)."""
+    from treemoe_spec_amd import _capi
+
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(len(counts))
+    e, rows = len(counts), sum(counts)
+    t, n, ki = rows // 2, 1024, 768
+    offsets, tiles = [0], []
+    for k, c in enumerate(counts):
+        tiles += [[k, offsets[k] + r0, min(64, c - r0), 0] for r0 in range(0, c, 64)]
+        offsets.append(offsets[-1] + c)
+    assert 2 * t <= 64 * e and len(tiles) * (n // 256) * 4 < 256    # the rule
+    print(f"narrow down {counts}", flush=True)
+    draw = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    hm, w2, gates = draw(rows, ki), draw(e, n, ki) * 0.1, torch.rand(rows, generator=g)
+    slots = torch.randperm(rows, generator=g).to(torch.int32)
+    as_dev = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    hmd, w2d, gd, sd, od, td = (hm.to(dev), w2.to(dev), gates.to(dev), slots.to(dev),
+                                as_dev(offsets), as_dev(tiles))
+    y = torch.full((4, rows + 1, n), 7.0, device=dev)
+    seg = ki // 4
+    _capi.call("tm_op1_prefill_gemm2", hmd.data_ptr(), w2d.data_ptr(), y.data_ptr(),
+               gd.data_ptr(), sd.data_ptr(), od.data_ptr(), td.data_ptr(), len(tiles), 4, t, n, ki,
+               e, _capi.TM_DTYPE_BF16, _capi.stream_of(dev))
+    out = y.double().cpu().reshape(-1)
+    assert torch.all(out[4 * rows * n:] == 7.0)      # nothing past the [4, rows, n] partials
+    out = out[:4 * rows * n].reshape(4, rows, n)
+    for k, c in enumerate(counts):
+        r = slice(offsets[k], offsets[k + 1])
+        for s in range(4):
+            a, w = (v[..., s * seg:(s + 1) * seg].double() for v in (hm[r], w2[k]))
+            gate = gates[slots[r].long()].double()[:, None]
+            ref, mag = gate * (a @ w.T), gate * (a.abs() @ w.abs().T)
+            assert torch.all((out[s, r] - ref).abs() <= (seg + 2) * 2.0 ** -24 * mag), (k, s)

@@ -21,14 +21,15 @@
 //            pipelined (PipeLoop): where the experts average 112 rows or more;
 //   Tile128  128 x 256 on 8 waves, three 48 KB stages;
 //   TileDec  64 x 128 on 4 waves, three 24 KB stages, so two workgroups share
-//            a CU: gate/up when the tile list leaves at most 16 rows per entry.
+//            a CU: gate/up when the tile list leaves at most 16 rows per entry,
+//            down where the other tile has too few jobs for the chip.
 // A tile whose M-tile holds fewer than BM real rows runs the MFMAs of the
 // 64-row parts that hold them only.
 //
 // Gate/up: B = BN / 2 rows of w1 and the same rows of w3, so each wave holds
 // the gate and up sums of the same outputs and applies SwiGLU in registers; h
 // is written row-major [sorted row, I] through an LDS-staged, coalesced store.
-// Down: B = 256 rows of w2 over one K segment; the gate weight multiplies the
+// Down: B = BN rows of w2 over one K segment; the gate weight multiplies the
 // fp32 sums before the store of the partial y[segment].
 //
 // M-tiles are BM consecutive rows of one expert in the compact expert-major
@@ -144,6 +145,7 @@ __device__ __forceinline__ int swz(int r, int c) {
   return r * C::PROW + ((c ^ ((r / C::RPB) & (C::CPR - 1))) << 4);
 }
 
+constexpr int kCUs = 256;
 constexpr int kXcds = 8;  // workgroup i runs on XCD i % 8
 constexpr int SBM = 8;    // super-block: M-tile slots (consecutive: mostly one expert) ..
 constexpr int SBN = 4;    // .. x column jobs, M fastest
@@ -923,7 +925,7 @@ tm_prefill_gemm1_routed_kernel(const uint16_t* __restrict__ x, const uint16_t* _
 
 // ---------------------------------------------------------------- down --
 // y[s, p, n] = gates_flat[slot(p)] * sum_{k in segment s} h[p, k] w2[e, n, k]
-// for the rows p of one M-tile and 256 output columns n.  The fp32 partials
+// for the rows p of one M-tile and BN output columns n.  The fp32 partials
 // go straight from the accumulators, 16 bytes per lane and store; a lane's
 // rows (one per accumulator row block) have their gates loaded before the K
 // loop.
@@ -1223,13 +1225,22 @@ extern "C" int tm_op1_prefill_gemm2(const void* h, const void* w2, float* y,
   if (klen < C::PBK || (klen % C::PBK) != 0 || H < C::PBN || (H % C::PBN) != 0) return TM_ERR_SHAPE;
   if (H * I * 2 >= (int64_t)kOOR || 2 * T * I * 2 >= (int64_t)kOOR) return TM_ERR_SHAPE;
   if (!aligned16(h) || !aligned16(w2) || !aligned16(y)) return TM_ERR_ALIGN;
-  const bool big = many_rows(T, E);  // the gate/up rule
-  const int rc = big ? launch_gemm2<Tile256>(h, w2, y, gates_flat, sorted_slots,
-                                               expert_offsets, tiles, max_tiles, split, T, H,
-                                               I, E, dtype, (hipStream_t)stream)
-                     : launch_gemm2<Tile128>(h, w2, y, gates_flat, sorted_slots, expert_offsets,
-                                             tiles, max_tiles, split, T, H, I, E, dtype,
-                                             (hipStream_t)stream);
+  // many_rows: the gate/up rule.  TileDec (twice the column jobs, two workgroups
+  // per CU) where the 128-row tile's jobs leave CUs without one and few experts
+  // exceed its 64 rows.  Down + combine on Tile128 against TileDec, four K
+  // segments, E = 8, I = 3584: H = 1024 (at most 144 jobs) T = 16 18.2 against
+  // 14.6 us, T = 64 18.9 / 15.1, T = 64 budget 4 19.8 / 14.1, T = 200 23.3 / 18.6;
+  // where the jobs fill the CUs, H = 4096, I = 14336, T = 64 budget 4 79.7 / 84.0.
+  const int64_t mt128 = std::min<int64_t>(max_tiles, mtile_bound<Tile128>(2 * T, E));
+  const bool dec = 2 * T <= 64 * E && mt128 * (H / C::PBN) * split < kCUs;
+  const int rc =
+      many_rows(T, E)
+          ? launch_gemm2<Tile256>(h, w2, y, gates_flat, sorted_slots, expert_offsets, tiles,
+                                  max_tiles, split, T, H, I, E, dtype, (hipStream_t)stream)
+      : dec ? launch_gemm2<TileDec>(h, w2, y, gates_flat, sorted_slots, expert_offsets, tiles,
+                                    max_tiles, split, T, H, I, E, dtype, (hipStream_t)stream)
+            : launch_gemm2<Tile128>(h, w2, y, gates_flat, sorted_slots, expert_offsets, tiles,
+                                    max_tiles, split, T, H, I, E, dtype, (hipStream_t)stream);
   if (rc) return rc;
   TM_HIP_CHECK_LAUNCH();
   return TM_OK;
