@@ -69,13 +69,25 @@ TILED_MIN_ROWS = 32           # tiled from this many rows per routed expert ..
 TILED_MIN_ROWS_WIDE = 8       # .. or from this many when inter >= TILED_WIDE_INTER
 TILED_WIDE_INTER = 3584
 
+# At a small hidden size the streaming kernels' work items are too short to
+# stream (gate/up: four K chunks, one per wave) and their latency shows, so the
+# tiled pair wins from two tokens on.  H=1024, I=3584, E=8, layer us, streaming /
+# tiled: B=8 T=1 26.8 / 27.7, T=2 36.0 / 30.7, T=4 51.6 / 38.0, T=24 57.5 / 42.1;
+# B=4 T=2 33.6 / 29.0, T=12 38.3 / 30.7; through the hook (routing in its own
+# launches) T=2 35.9 / 35.3, T=4 51.6 / 43.4.  H=4096, I=3584: T=4 111.4 / 110.8.
+TILED_SMALL_HIDDEN = 1024
+
 
 def uses_tiled_gemms(num_tokens: int, expert_budget: int, num_experts: int,
-                     inter: int = 0) -> bool:
-    """True when the average rows per routed expert reach TILED_MIN_ROWS, or
-    TILED_MIN_ROWS_WIDE for an intermediate size of TILED_WIDE_INTER or more."""
+                     inter: int = 0, hidden: int = 0) -> bool:
+    """True when the average rows per routed expert reach TILED_MIN_ROWS, or for
+    an intermediate size of TILED_WIDE_INTER or more TILED_MIN_ROWS_WIDE, or
+    there two tokens where the hidden size (0: unknown) is at most
+    TILED_SMALL_HIDDEN."""
     active = min(expert_budget, num_experts)
     if 2 * num_tokens >= TILED_MIN_ROWS * active:
+        return True
+    if 0 < hidden <= TILED_SMALL_HIDDEN and inter >= TILED_WIDE_INTER and num_tokens >= 2:
         return True
     return inter >= TILED_WIDE_INTER and 2 * num_tokens >= TILED_MIN_ROWS_WIDE * active
 
@@ -411,10 +423,11 @@ SELF_ROUTED_MAX_EXPERTS = 16
 _SELF_ROUTED_MAX_BLOCKS = 256      # compact_block_capacity(2T, B, BM)
 
 
-def self_routed(num_tokens: int, expert_budget: int, num_experts: int, inter: int) -> bool:
+def self_routed(num_tokens: int, expert_budget: int, num_experts: int, inter: int,
+                hidden: int = 0) -> bool:
     """True when tree_moe_forward (without a precomputed routing) runs the
     routing inside the gate/up launch: the tiled GEMMs at few tokens."""
-    return (uses_tiled_gemms(num_tokens, expert_budget, num_experts, inter)
+    return (uses_tiled_gemms(num_tokens, expert_budget, num_experts, inter, hidden)
             and num_tokens <= SELF_ROUTED_MAX_TOKENS
             and num_experts <= SELF_ROUTED_MAX_EXPERTS
             and compact_block_capacity(2 * num_tokens, expert_budget, BM)
@@ -460,8 +473,8 @@ def _forward(x, w1, w2, w3, router_weight, node_accept_prob, expert_budget, out,
         raise ValueError("expected w1, w3 [E, I, H] and w2 [E, H, I] matching x [T, H]")
     if hidden % 256 != 0 or inter % 256 != 0:
         raise ValueError("hidden and intermediate sizes must be multiples of 256")
-    tiled = uses_tiled_gemms(n, expert_budget, e, inter)
-    if routing is None and self_routed(n, expert_budget, e, inter):
+    tiled = uses_tiled_gemms(n, expert_budget, e, inter, hidden)
+    if routing is None and self_routed(n, expert_budget, e, inter, hidden):
         # router, then the gate/up launch that also routes and buckets
         _check_router(x, router_weight)
         stream = _capi.stream_of(x.device)
