@@ -424,14 +424,12 @@ constexpr int kSampWaves = kSampThreads / 64;
 // gfx950, no dearer than fmaxf): a NaN logit, a +inf one (inf - inf) or a
 // row of -inf makes the row NaN, as torch.softmax's.  (A NaN test on every
 // entry instead cost ~4 us per config-4 call: the walk is VALU-bound.)
-__device__ __forceinline__ float clamp_min_nan(float x, float lo) {
-  return x != x ? x : fmaxf(x, lo);
-}
-__device__ __forceinline__ float clamp_max_nan(float x, float hi) {
-  return x != x ? x : fminf(x, hi);
-}
 __device__ __forceinline__ float max_nan(float a, float b) {
   return __builtin_elementwise_maximum(a, b);
+}
+__device__ __forceinline__ float clamp_min_nan(float x, float lo) { return max_nan(x, lo); }
+__device__ __forceinline__ float clamp_max_nan(float x, float hi) {
+  return x != x ? x : fminf(x, hi);
 }
 // e^(x - m) for the sampling softmax, given ml = m log2(e): the hardware
 // exponential v_exp_f32 of fma(x, log2(e), -ml).  The walk is VALU-bound
@@ -474,10 +472,14 @@ __device__ __forceinline__ float logit_at(const void* logits, int64_t at) {
 
 
 // ----------------------------------------------- sampling, in registers --
-// For V <= kSampThreads * R: thread t owns residual entries
-// [t * R, t * R + R) in registers, so a row pass issues every load of the
-// thread at once instead of one dependent load per loop trip, and the bonus
-// scan is a shuffle scan.  Entries at or past V hold 0 (-inf as logits).
+// For V <= kSampThreads * R: thread t owns R residual entries in registers, so a
+// row pass issues every load of the thread at once instead of one dependent
+// load per loop trip.  The entries are R / 4 groups of four, kSampThreads groups
+// apart (samp_entry): a wave's load of one group per lane is 1 KB of consecutive
+// floats.  (With R consecutive entries per thread every lane's 16 bytes lay in
+// a cache line of their own, and passing those lines through the one CU took
+// longer than the arithmetic: a sampling step at V = 32000, float32 logits, 64
+// nodes 74 -> 61 us through the Python API.)  Entries at or past V hold 0 (-inf as logits).
 // Reductions are in a fixed order: the thread's entries in index order, then
 // a butterfly over the wave, then the 16 wave values in wave order.
 struct SampRegShared {
@@ -565,54 +567,63 @@ __device__ __forceinline__ float block_reduce_fast(float v, bool is_max, SampReg
   return r;
 }
 
-// x[i] = element lo + i of a row of `kDtype` (fill beyond V); 16-byte loads
-// when the row is aligned and the thread's range lies inside [0, V).
+// Vocabulary index of this thread's entry i of the kSampThreads * R entries
+// from `first` on.  It ascends with i.
+__device__ __forceinline__ int samp_entry(int first, int i) {
+  return first + ((i >> 2) * kSampThreads + (int)threadIdx.x) * 4 + (i & 3);
+}
+// The thread that owns entry `at` (counted from a multiple of 4 kSampThreads),
+// and its i there.
+__device__ __forceinline__ int samp_owner(int at) { return (at >> 2) % kSampThreads; }
+__device__ __forceinline__ int samp_index(int at) {
+  return (at >> 2) / kSampThreads * 4 + (at & 3);
+}
+
+// x[i] = this thread's entry i from `first` on of a row of `kDtype` (fill
+// beyond V); one vector load per group of four when the row is aligned and the
+// group lies inside [0, V).
 template <int kDtype, int R>
-__device__ __forceinline__ void load_range(const void* row, int lo, int V, bool vec, float fill,
+__device__ __forceinline__ void load_range(const void* row, int first, int V, bool vec, float fill,
                                            float (&x)[R]) {
-  if (vec && lo + R <= V) {
-    if (kDtype == TM_DTYPE_F32) {
-      const float4* p = reinterpret_cast<const float4*>(reinterpret_cast<const float*>(row) + lo);
 #pragma unroll
-      for (int j = 0; j < R / 4; ++j) {
-        const float4 f = p[j];
-        x[4 * j] = f.x;
-        x[4 * j + 1] = f.y;
-        x[4 * j + 2] = f.z;
-        x[4 * j + 3] = f.w;
+  for (int j = 0; j < R; j += 4) {
+    const int at = samp_entry(first, j);
+    if (vec && at + 4 <= V) {
+      if (kDtype == TM_DTYPE_F32) {
+        const float4 f = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(row) + at);
+        x[j] = f.x;
+        x[j + 1] = f.y;
+        x[j + 2] = f.z;
+        x[j + 3] = f.w;
+      } else {
+        const uint2 u =
+            *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(row) + at);
+        x[j] = __uint_as_float(u.x << 16);
+        x[j + 1] = __uint_as_float(u.x & 0xffff0000u);
+        x[j + 2] = __uint_as_float(u.y << 16);
+        x[j + 3] = __uint_as_float(u.y & 0xffff0000u);
       }
     } else {
-      const uint4* p = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(row) + lo);
 #pragma unroll
-      for (int j = 0; j < R / 8; ++j) {
-        const uint4 u = p[j];
-        const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          x[8 * j + 2 * k] = __uint_as_float(w[k] << 16);
-          x[8 * j + 2 * k + 1] = __uint_as_float(w[k] & 0xffff0000u);
-        }
-      }
+      for (int k = 0; k < 4; ++k)
+        x[j + k] = at + k < V ? logit_at<kDtype>(row, at + k) : fill;
     }
-  } else {
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-      x[i] = (lo + i < V) ? logit_at<kDtype>(row, lo + i) : fill;
   }
 }
 
 template <int R>
-__device__ __forceinline__ void store_range(float* dst, int lo, int V, bool vec,
+__device__ __forceinline__ void store_range(float* dst, int first, int V, bool vec,
                                             const float (&x)[R]) {
-  if (vec && lo + R <= V) {
-    float4* p = reinterpret_cast<float4*>(dst + lo);
 #pragma unroll
-    for (int j = 0; j < R / 4; ++j)
-      p[j] = make_float4(x[4 * j], x[4 * j + 1], x[4 * j + 2], x[4 * j + 3]);
-  } else {
+  for (int j = 0; j < R; j += 4) {
+    const int at = samp_entry(first, j);
+    if (vec && at + 4 <= V) {
+      *reinterpret_cast<float4*>(dst + at) = make_float4(x[j], x[j + 1], x[j + 2], x[j + 3]);
+    } else {
 #pragma unroll
-    for (int i = 0; i < R; ++i)
-      if (lo + i < V) dst[lo + i] = x[i];
+      for (int k = 0; k < 4; ++k)
+        if (at + k < V) dst[at + k] = x[j + k];
+    }
   }
 }
 
@@ -657,7 +668,7 @@ __device__ __forceinline__ int block_argmax(float v, int idx, SampRegShared& sh,
   return bi;
 }
 
-// One thread's part of the exponential race over entries lo .. lo + R - 1
+// One thread's part of the exponential race over its R entries from `first` on
 // (x: residual entries, e: the exponentials; entries at or past V skipped):
 // the first of its largest x[i] / e[i] (IEEE division, as torch's div).  A
 // NaN ratio never wins here; the residual is NaN-free or all NaN (a NaN logit
@@ -667,15 +678,16 @@ __device__ __forceinline__ int block_argmax(float v, int idx, SampRegShared& sh,
 // probability, not a probability, could leave a partly NaN residual, whose
 // NaN entries this race skips where torch.argmax would take the first.
 template <int R>
-__device__ __forceinline__ void race_chunk(const float (&x)[R], const float (&e)[R], int lo,
+__device__ __forceinline__ void race_chunk(const float (&x)[R], const float (&e)[R], int first,
                                            int V, float& best, int& at) {
 #pragma unroll
   for (int i = 0; i < R; ++i) {
-    if (lo + i < V) {
+    const int idx = samp_entry(first, i);
+    if (idx < V) {
       const float t = x[i] / e[i];
       if (t > best) {  // indices ascend: ties keep the first
         best = t;
-        at = lo + i;
+        at = idx;
       }
     }
   }
@@ -697,7 +709,6 @@ tm_sample_walk_reg_kernel(const void* __restrict__ logits, int N, int V, int64_t
   __shared__ SampRegShared sh;
   __shared__ SampTree tree;
   const int tid = threadIdx.x;
-  const int lo = tid * R;
   const bool staged = N <= kSampStage && num_edges <= kSampStage;
   if (staged)
     stage_tree(tree, N, V, tokens, child_start, child_count, child_list, num_edges, uniforms, q,
@@ -712,7 +723,7 @@ tm_sample_walk_reg_kernel(const void* __restrict__ logits, int N, int V, int64_t
     // r = softmax(logits[node] / temperature)
     const char* row = reinterpret_cast<const char*>(logits) +
                       (int64_t)node * row_stride * (kDtype == TM_DTYPE_F32 ? 4 : 2);
-    load_range<kDtype, R>(row, lo, V, vec_logits != 0, -INFINITY, r);
+    load_range<kDtype, R>(row, 0, V, vec_logits != 0, -INFINITY, r);
     float m = -INFINITY;
     if (unit_t) {  // x / 1 = x: no division at temperature 1
 #pragma unroll
@@ -746,12 +757,12 @@ tm_sample_walk_reg_kernel(const void* __restrict__ logits, int N, int V, int64_t
       const int c = ct.x, tok = ct.y;
       if (c < 0) continue;
       // the owner of entry tok decides; tid 0 answers for an out-of-vocabulary token
-      if (tok >= 0 ? tok / R == tid : tid == 0) {
+      if (tok >= 0 ? samp_owner(tok) == tid : tid == 0) {
         int ok = 0;
         if (tok >= 0) {
           float rv = 0.0f;
 #pragma unroll
-          for (int i = 0; i < R; ++i) rv = (lo + i == tok) ? r[i] : rv;
+          for (int i = 0; i < R; ++i) rv = (i == samp_index(tok)) ? r[i] : rv;
           ok = sample_accept(staged, tree, c, tok, rv, uniforms, q, q_stride);
         }
         sh.flag = ok;
@@ -770,8 +781,8 @@ tm_sample_walk_reg_kernel(const void* __restrict__ logits, int N, int V, int64_t
 #pragma unroll
       for (int b = 0; b < R; b += kQB) {
         float qc[kQB];
-        load_range<TM_DTYPE_F32, kQB>(q + (int64_t)c * q_stride, lo + b, V, vec_q != 0, 0.0f,
-                                      qc);
+        load_range<TM_DTYPE_F32, kQB>(q + (int64_t)c * q_stride, b * kSampThreads, V, vec_q != 0,
+                                      0.0f, qc);
 #pragma unroll
         for (int i = 0; i < kQB; ++i) {
           r[b + i] = clamp_min_nan(r[b + i] - qc[i], 0.0f);
@@ -796,10 +807,10 @@ tm_sample_walk_reg_kernel(const void* __restrict__ logits, int N, int V, int64_t
 
   // bonus: the exponential race, argmax_j r[j] / e[j], first maximum
   float e[R];
-  load_range<TM_DTYPE_F32, R>(bonus_exp, lo, V, vec_e != 0, 1.0f, e);
+  load_range<TM_DTYPE_F32, R>(bonus_exp, 0, V, vec_e != 0, 1.0f, e);
   float best = -1.0f;
   int at = INT_MAX;
-  race_chunk<R>(r, e, lo, V, best, at);
+  race_chunk<R>(r, e, 0, V, best, at);
   const int won = block_argmax(best, at, sh, phase);
   const int bonus = won == INT_MAX ? 0 : won;  // an all-NaN race: torch.argmax's index 0
   if (tid == 0) {
@@ -807,7 +818,7 @@ tm_sample_walk_reg_kernel(const void* __restrict__ logits, int N, int V, int64_t
     result[1] = count;
     result[2] = node;
   }
-  store_range<R>(res, lo, V, vec_res != 0, r);
+  store_range<R>(res, 0, V, vec_res != 0, r);
   for (int i = count + tid; i < N; i += kSampThreads) {
     accepted_slots[i] = -1;
     accepted_tokens[i] = -1;
@@ -816,10 +827,9 @@ tm_sample_walk_reg_kernel(const void* __restrict__ logits, int N, int V, int64_t
 
 // ------------------------------------------------- sampling, in tiles --
 // For V > kSampRegMax: the residual lives in `res` and every pass walks the
-// row in tiles of kSampTile entries; thread t owns entries
-// [tile * kSampTile + t * kSampTR, + kSampTR) of every tile, so it issues a
-// tile's loads at once and only ever reads back residual entries it wrote
-// itself.  Sums accumulate over the thread's entries tile by tile, then as in
+// row in tiles of kSampTile entries; a thread owns kSampTR entries of every tile
+// (samp_entry), so it issues a tile's loads at once and only ever reads back
+// residual entries it wrote itself.  Sums accumulate over the thread's entries tile by tile, then as in
 // the register kernel; the bonus race runs over the tiles in order.
 constexpr int kSampTR = 32;
 constexpr int kSampTile = kSampThreads * kSampTR;
@@ -862,7 +872,7 @@ tm_sample_walk_tiled_kernel(const void* __restrict__ logits, int N, int V, int64
     float m = -INFINITY;
     for (int tl = 0; tl < tiles; ++tl) {
       float x[kSampTR];
-      load_range<kDtype, kSampTR>(row, tl * kSampTile + tid * kSampTR, V, vl, -INFINITY, x);
+      load_range<kDtype, kSampTR>(row, tl * kSampTile, V, vl, -INFINITY, x);
 #pragma unroll
       for (int i = 0; i < kSampTR; ++i) m = max_nan(m, x[i]);
     }
@@ -873,7 +883,7 @@ tm_sample_walk_tiled_kernel(const void* __restrict__ logits, int N, int V, int64
     // the exponentials go to res, then one pass scales them by 1 / sum
     float s = 0.0f;
     for (int tl = 0; tl < tiles; ++tl) {
-      const int lo = tl * kSampTile + tid * kSampTR;
+      const int lo = tl * kSampTile;
       float x[kSampTR];
       load_range<kDtype, kSampTR>(row, lo, V, vl, -INFINITY, x);
       if (unit_t) {
@@ -893,7 +903,7 @@ tm_sample_walk_tiled_kernel(const void* __restrict__ logits, int N, int V, int64
     }
     const float rs = 1.0f / block_reduce_fast(s, false, sh, phase);
     for (int tl = 0; tl < tiles; ++tl) {
-      const int lo = tl * kSampTile + tid * kSampTR;
+      const int lo = tl * kSampTile;
       float x[kSampTR];
       load_range<TM_DTYPE_F32, kSampTR>(res, lo, V, vr, 0.0f, x);
 #pragma unroll
@@ -910,7 +920,7 @@ tm_sample_walk_tiled_kernel(const void* __restrict__ logits, int N, int V, int64
       const int c = ct.x, tok = ct.y;
       if (c < 0) continue;
       // the thread that wrote res[tok] decides; tid 0 for an out-of-vocabulary token
-      if (tok >= 0 ? (tok % kSampTile) / kSampTR == tid : tid == 0) {
+      if (tok >= 0 ? samp_owner(tok) == tid : tid == 0) {
         int ok = 0;
         if (tok >= 0) ok = sample_accept(staged, tree, c, tok, res[tok], uniforms, q, q_stride);
         sh.flag = ok;
@@ -924,7 +934,7 @@ tm_sample_walk_tiled_kernel(const void* __restrict__ logits, int N, int V, int64
       const float* qrow = q + (int64_t)c * q_stride;
       float part = 0.0f;
       for (int tl = 0; tl < tiles; ++tl) {
-        const int lo = tl * kSampTile + tid * kSampTR;
+        const int lo = tl * kSampTile;
         float x[kSampTR], qc[kSampTR];
         load_range<TM_DTYPE_F32, kSampTR>(res, lo, V, vr, 0.0f, x);
         load_range<TM_DTYPE_F32, kSampTR>(qrow, lo, V, vq, 0.0f, qc);
@@ -937,7 +947,7 @@ tm_sample_walk_tiled_kernel(const void* __restrict__ logits, int N, int V, int64
       }
       const float rtot = 1.0f / clamp_min_nan(block_reduce_fast(part, false, sh, phase), 1e-20f);
       for (int tl = 0; tl < tiles; ++tl) {
-        const int lo = tl * kSampTile + tid * kSampTR;
+        const int lo = tl * kSampTile;
         float x[kSampTR];
         load_range<TM_DTYPE_F32, kSampTR>(res, lo, V, vr, 0.0f, x);
 #pragma unroll
@@ -962,7 +972,7 @@ tm_sample_walk_tiled_kernel(const void* __restrict__ logits, int N, int V, int64
   float best = -1.0f;
   int at = INT_MAX;
   for (int tl = 0; tl < tiles; ++tl) {
-    const int lo = tl * kSampTile + tid * kSampTR;
+    const int lo = tl * kSampTile;
     float x[kSampTR], e[kSampTR];
     load_range<TM_DTYPE_F32, kSampTR>(res, lo, V, vr, 0.0f, x);
     load_range<TM_DTYPE_F32, kSampTR>(bonus_exp, lo, V, vec_e != 0, 1.0f, e);
