@@ -80,9 +80,14 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
 }
 
 // Stage layout: thread t stages keys 4 * quad + r (r = 0..3) at head-dim
-// elements 8 * part .. +7, with quad = (t & 3) + 4 * (t >> 6) and
-// part = (t >> 2) & 15; this order keeps both the K row writes and the
-// transposed V writes free of LDS bank conflicts.
+// elements 8 * part .. +7, with part = t & 15 and quad = t >> 4: 16 consecutive
+// lanes read one key's 256 bytes.  (With four keys in four consecutive lanes,
+// every lane's 16 bytes of a load lay in another cache line than its
+// neighbours', which took the address path four times as long.)  In a row of
+// V^T the 16 key quads are stored at quad ^ 4 (part / 4), so that a wave's
+// transposed writes (16 parts x 4 quads, rows 8 parts apart 16 banks apart) are
+// spread over the banks; for a fragment of head-dim tile ht that is the
+// constant 4 ht.
 struct Stage {
   u32x4_t k[4];
   u32x4_t v[4];
@@ -143,7 +148,7 @@ __device__ __forceinline__ void store_stage(uint8_t* buf, int quad, int part, co
     u32x2_t pk;
     pk.x = __builtin_amdgcn_perm(st.v[1][w], st.v[0][w], sel);
     pk.y = __builtin_amdgcn_perm(st.v[3][w], st.v[2][w], sel);
-    *reinterpret_cast<u32x2_t*>(vl + (8 * part + j) * kVStride + quad * 8) = pk;
+    *reinterpret_cast<u32x2_t*>(vl + (8 * part + j) * kVStride + (quad ^ (4 * (part >> 2))) * 8) = pk;
   }
 }
 
@@ -285,7 +290,9 @@ __device__ __forceinline__ void attend_stage(const AttnParams& p, const uint8_t*
       b.w = pack_bf16(sc[kt][8 * m + 6], sc[kt][8 * m + 7]);
 #pragma unroll
       for (int ht = 0; ht < kHD / 32; ++ht) {
-        const uint8_t* vr = vl + (32 * ht + c32) * kVStride + (32 * kt + 16 * m + 4 * half) * 2;
+        // key quads 8 kt + 4 m + half and + 2, at their place in rows of tile ht
+        const uint8_t* vr =
+            vl + (32 * ht + c32) * kVStride + (((8 * kt + 4 * m) ^ (4 * ht)) + half) * 8;
         const u32x2_t lo = *reinterpret_cast<const u32x2_t*>(vr);
         const u32x2_t hi = *reinterpret_cast<const u32x2_t*>(vr + 16);
         const u32x4_t a = {lo.x, lo.y, hi.x, hi.y};
@@ -321,8 +328,8 @@ __global__ void __launch_bounds__(kThreads, 2) tm_tree_attn_kernel(AttnParams p)
   const bool lead = chunk < p.pre_chunks;
   const int c0 = (lead ? 0 : p.split) + (lead ? chunk : chunk - p.pre_chunks) * p.chunk_len;
   const int c1 = min(c0 + p.chunk_len, lead ? p.split : s_total);
-  const int quad = (tid & 3) + 4 * (tid >> 6);
-  const int part = (tid >> 2) & 15;
+  const int quad = tid >> 4;
+  const int part = tid & 15;
   const int64_t head_off = (int64_t)kvhead * kHD + part * 8;
 
   // block-table entries of the chunk's prefix keys; the workgroups of row
