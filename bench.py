@@ -202,8 +202,8 @@ def kernel_breakdown(m, inp, reps: int) -> dict:
     res = {}
     for k, name in enumerate(names):
         res[name] = median([ev[r][k].elapsed_time(ev[r][k + 1]) for r in range(reps)])
-    res["tiled"] = m.uses_tiled_gemms(n, budget, e, inter)
-    res["self_routed"] = m.self_routed(n, budget, e, inter)
+    res["tiled"] = m.uses_tiled_gemms(n, budget, e, inter, hidden)
+    res["self_routed"] = m.self_routed(n, budget, e, inter, hidden)
     res["max_tiles"] = m.compact_block_limit(2 * n, budget, m.TILE_M)
     return res
 
