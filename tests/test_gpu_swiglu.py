@@ -1,0 +1,71 @@
+"""SwiGLU of the tiled gate/up over the whole range of the gate's pre-activation,
+against float64, on each of its tiles.
+
+A token's first feature is its pre-activation a and the w3 rows scale the second
+to b, so a and b are exact.  h = silu(a) b carries, relative to |h|: the rounding
+to 16 bits (2^-9 in bf16, 2^-12 in fp16, plus half its smallest subnormal) and
+the fp32 exponential, sum, division and product.  The exponential's error is
+that of a log2(e) rounded to fp32, at most |a| 2^-24 relative, plus one unit
+(2^-23) of the instruction; the other three operations round once, 2^-24 each.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# e^-a overflows fp32 below this: silu is then -0
+OVERFLOW = -88.72
+TILES = [("256 rows", 2, 14), ("128 rows", 8, 14), ("64 rows", 8, 52)]
+
+
+def _gate_up(tile, experts, max_tiles, a, c, b, dtype):
+    """(h, a, c per row): experts 0 and 1 hold every token, the others none."""
+    from treemoe_spec_amd import _capi
+
+    dev = torch.device("cuda")
+    t, h, i = a.numel(), 64, b.numel()
+    rows = 2 * t
+    # the rule of tm_op1_prefill_gemm1: 256 rows, else 64 rows, else 128
+    assert tile == ("256 rows" if rows >= 112 * experts else
+                    "64 rows" if rows <= 16 * max_tiles else "128 rows")
+    x = torch.zeros(t, h)
+    x[:, 0], x[:, 1] = a, c
+    w1, w3 = torch.zeros(experts, i, h), torch.zeros(experts, i, h)
+    w1[:, :, 0], w3[:, :, 1] = 1.0, b
+    slots = torch.cat([torch.arange(0, rows, 2), torch.arange(1, rows, 2)]).to(torch.int32)
+    offsets = torch.tensor([0, t] + [rows] * (experts - 1), dtype=torch.int32)
+    tiles = [[e, e * t + r, min(64, t - r), 0] for e in range(2) for r in range(0, t, 64)]
+    assert len(tiles) <= max_tiles
+    tiles = torch.tensor(tiles + [[-1, 0, 0, 0]] * (max_tiles - len(tiles)), dtype=torch.int32)
+    xd, w1d, w3d = (v.to(device=dev, dtype=dtype) for v in (x, w1, w3))
+    sd, od, td = slots.to(dev), offsets.to(dev), tiles.to(dev)
+    hd = torch.empty(rows, i, dtype=dtype, device=dev)
+    _capi.call("tm_op1_prefill_gemm1", xd.data_ptr(), w1d.data_ptr(), w3d.data_ptr(),
+               hd.data_ptr(), sd.data_ptr(), od.data_ptr(), td.data_ptr(), max_tiles, t, h, i,
+               experts, _capi.TM_DTYPE_BF16 if dtype == torch.bfloat16 else _capi.TM_DTYPE_F16,
+               _capi.stream_of(dev))
+    token = slots.long() >> 1
+    return hd.cpu(), x[token, 0].double()[:, None], x[token, 1].double()[:, None]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tile,experts,max_tiles", TILES)
+def test_swiglu_range_matches_float64(tile, experts, max_tiles, dtype):
+    print(f"swiglu {tile} {dtype}", flush=True)
+    a = torch.cat([torch.arange(-100.0, 100.25, 0.5), torch.zeros(1)])   # exact in 16 bits
+    # b over the powers of two that the type holds
+    powers = [-60, -10, 0, 8, 30, 60, 90, 120] if dtype == torch.bfloat16 else [-8, -4, -1, 0, 1, 4]
+    b = torch.tensor([2.0 ** powers[n % len(powers)] for n in range(256)])
+    h, av, _ = _gate_up(tile, experts, max_tiles, a, torch.ones_like(a), b, dtype)
+    out = h.double()
+    ref = av * torch.sigmoid(av) * b.double()
+    info = torch.finfo(dtype)
+    assert ref.abs().max() < info.max
+    half_ulp = info.eps / 2
+    tol = (half_ulp + (av.abs() + 5.0) * 2.0 ** -24) * ref.abs() + info.smallest_normal * half_ulp
+    tol = torch.where(av < OVERFLOW, ref.abs(), tol)
+    bad = (out - ref).abs() > tol
+    assert not bad.any(), (av.expand_as(ref)[bad][:4], out[bad][:4], ref[bad][:4])

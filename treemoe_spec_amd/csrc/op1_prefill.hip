@@ -625,12 +625,16 @@ __device__ __forceinline__ uint8_t* h_stage(const Stages& sb, int m) {
   return base + (m % C::HROWS) * C::HSTRIDE;
 }
 
-// silu(a) b in fp32, silu(a) = a / (1 + e^-a): the hardware exponential and
-// reciprocal (each within one unit of 2^-23 before the result is rounded to 8
-// or 11 bits); the IEEE division took ten operations per value.  a = -inf and
-// NaN give NaN, e^-a = inf gives -0, as the division did.
+// silu(a) b in fp32, silu(a) = a / (1 + e^-a), as the weight-streaming gate/up
+// computes it.  __expf rounds a log2(e) before the base-2 exponential, so its
+// relative error grows with |a|, about |a| 2^-24: 5e-6 where e^-a overflows, far
+// below the 2^-9 (bf16) or 2^-12 (fp16) of the rounding of h.  The division is
+// the IEEE one: the reciprocal instruction flushes a subnormal result, which
+// made silu(a) 0 for a between -88.7 and -87.3, where it is a normal number
+// (same box, one layer: T = 517 587 -> 593 us, T = 2048 1413 -> 1427, T = 6011
+// 3535 -> 3570).
 __device__ __forceinline__ float swiglu(float a, float b) {
-  return (a * __builtin_amdgcn_rcpf(1.0f + __expf(-a))) * b;
+  return (a / (1.0f + __expf(-a))) * b;
 }
 
 // The MFMAs and the epilogue of one gate/up tile with M accumulator tiles
