@@ -69,3 +69,20 @@ def test_swiglu_range_matches_float64(tile, experts, max_tiles, dtype):
     tol = torch.where(av < OVERFLOW, ref.abs(), tol)
     bad = (out - ref).abs() > tol
     assert not bad.any(), (av.expand_as(ref)[bad][:4], out[bad][:4], ref[bad][:4])
+
+
+@pytest.mark.parametrize("tile,experts,max_tiles", TILES)
+def test_fp16_h_is_rounded_once(tile, experts, max_tiles):
+    """fp16 h where silu(a) = a exactly (e^-a below half a unit of 1) and b is a product of two
+    11-bit values: the 33-bit product a b rounded once to fp16, not to fp32 first."""
+    print(f"fp16 rounding {tile}", flush=True)
+    g = torch.Generator().manual_seed(5)
+    a = (18.0 + 40.0 * torch.rand(402, generator=g)).half().float()
+    c = (1.0 + torch.rand(402, generator=g)).half().float()
+    b = (1.0 + torch.rand(256, generator=g)).half().float()
+    h, av, cv = _gate_up(tile, experts, max_tiles, a, c, b, torch.float16)
+    exact = (av * cv * b.double()).numpy()
+    once = torch.from_numpy(exact.astype("float16"))
+    twice = torch.from_numpy(exact.astype("float32").astype("float16"))
+    assert (once != twice).sum() >= 8      # the values that tell the two apart
+    assert torch.equal(h, once), ((h != once).sum(), (h != twice).sum())

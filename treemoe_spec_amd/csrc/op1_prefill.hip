@@ -122,19 +122,22 @@ __device__ __forceinline__ f32x16_t pmfma(u32x4_t x, u32x4_t w, f32x16_t c) {
 // First of the four output columns that accumulator values 4 q .. 4 q + 3 hold.
 __device__ __forceinline__ int acc_col(int q, int lane) { return 8 * q + 4 * (lane >> 5); }
 
-// Four fp32 values to the 16-bit type, round to nearest even, packed in order
-// (bf16: v_cvt_pk_bf16_f32, one instruction per pair).
+// Two fp32 values to the 16-bit type, round to nearest even, packed in order
+// (bf16: v_cvt_pk_bf16_f32).  fp16 converts one value at a time, as Half16 does:
+// the product that ends a value then fuses with its conversion (v_fma_mixlo_f16,
+// v_fma_mixhi_f16) and is rounded once, where a conversion of the pair rounds
+// the fp32 product again.
 typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 template <int DT>
 __device__ __forceinline__ uint32_t pack16(float lo, float hi) {
-  const f32x2_t v = {lo, hi};
-  if constexpr (DT == TM_DTYPE_F16)
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
-  else
+  if constexpr (DT == TM_DTYPE_F16) {
+    return (uint32_t)tm_f32_to_f16(lo) | ((uint32_t)tm_f32_to_f16(hi) << 16);
+  } else {
+    const f32x2_t v = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
+  }
 }
 
 // Byte offset in a swizzled tile of logical chunk c (16 B) of row r: chunk c
