@@ -66,6 +66,12 @@ const char* tm_status_string(int code);
  * No reference counterpart: a utility of this ABI. */
 int tm_host_device_pointer(void* host, void** device);
 
+/* *id = 0, or, while a graph capture is under way on `stream`, one more than
+ * the capture's id (hipStreamGetCaptureInfo): the same for every call that one
+ * capture records.  For callers that keep device buffers between calls.
+ * No reference counterpart: a utility of this ABI. */
+int tm_stream_capture_id(void* stream, uint64_t* id);
+
 /* ---------------------------------------------------------------- op1 -- */
 
 /* `dtype` of the op1 entry points is the type of x, the weights, h and the

@@ -1,0 +1,75 @@
+"""CPU: which device buffers tree attention keeps between calls.  The packed mask
+words and the chunk partials belong to one stream (the partials to one thread
+too), and a graph capture gets its own."""
+
+from __future__ import annotations
+
+import threading
+
+import pytest
+import torch
+
+from treemoe_spec_amd.kernels import tree_attention as ta
+
+CPU = torch.device("cpu")
+
+
+@pytest.fixture()
+def packs(monkeypatch):
+    """The (stream, capture) under which masks are packed, and the packs done."""
+    state = {"stream": 0, "capture": 0, "done": []}
+    monkeypatch.setattr(ta, "_mask_cache", {})
+    monkeypatch.setattr(ta, "call", lambda name, *a: state["done"].append((name, a[-1])))
+    monkeypatch.setattr(ta._capi, "stream_of", lambda dev: state["stream"])
+    monkeypatch.setattr(ta, "_capture_id", lambda stream: state["capture"], raising=False)
+    return state
+
+
+def test_mask_words_are_packed_per_stream_and_capture(packs):
+    mask = torch.eye(3, dtype=torch.bool)
+    first = ta.pack_tree_mask(mask)
+    assert ta.pack_tree_mask(mask) is first and len(packs["done"]) == 1
+    packs["stream"] = 7
+    second = ta.pack_tree_mask(mask)
+    assert second is not first and packs["done"][-1] == ("tm_tree_mask_pack", 7)
+    # inside a capture: packed again by the capture, once for all its layers
+    packs["capture"] = 1
+    captured = ta.pack_tree_mask(mask)
+    assert captured is not second and len(packs["done"]) == 3
+    assert ta.pack_tree_mask(mask) is captured and len(packs["done"]) == 3
+    packs["capture"] = 2
+    assert ta.pack_tree_mask(mask) is not captured
+    # and eager calls go on with their own
+    packs["capture"] = 0
+    assert ta.pack_tree_mask(mask) is second and len(packs["done"]) == 4
+    mask[2, 0] = True
+    assert ta.pack_tree_mask(mask) is not second
+
+
+def test_workspace_belongs_to_a_stream_and_a_thread(monkeypatch):
+    monkeypatch.setattr(ta, "_ws_cache", {})
+    a = ta._workspace(100, CPU, 1, 0)
+    assert ta._workspace(60, CPU, 1, 0) is a          # reused in stream order
+    assert ta._workspace(100, CPU, 2, 0) is not a
+    other = []
+    t = threading.Thread(target=lambda: other.append(ta._workspace(100, CPU, 1, 0)))
+    t.start()
+    t.join()
+    assert other[0] is not a
+    assert ta._workspace(200, CPU, 1, 0).numel() == 200      # grown
+    assert ta._workspace(0, CPU, 1, 0) is None
+
+
+def test_workspace_of_a_capture_is_not_kept(monkeypatch):
+    monkeypatch.setattr(ta, "_ws_cache", {})
+    kept = ta._workspace(100, CPU, 1, 0)
+    inside = ta._workspace(100, CPU, 1, 5)
+    assert inside is not kept and ta._workspace(100, CPU, 1, 5) is not inside
+    assert ta._workspace(100, CPU, 1, 0) is kept
+
+
+def test_kept_workspaces_are_bounded(monkeypatch):
+    monkeypatch.setattr(ta, "_ws_cache", {})
+    for stream in range(1, 200):
+        ta._workspace(16, CPU, stream, 0)
+    assert len(ta._ws_cache) <= 32

@@ -34,6 +34,7 @@ SIGNATURES: dict[str, list] = {
     "tm_op4_kv_commit": [P, P, I64, I64, I64, I64, I64, I64, I64, P, P, P, I64, P, I64, I64,
                          I64, P, P],
     "tm_host_device_pointer": [P, P],
+    "tm_stream_capture_id": [P, P],
     "tm_op4_argmax_walk_noalloc": [P, I32, I64, I64, I64, P, P, P, P, I64, I64, I32, P, P, P,
                                    P, P],
     "tm_op4_rep_penalty": [P, I32, I64, I64, I64, P, I64, F32, P, I64, P],

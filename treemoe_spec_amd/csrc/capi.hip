@@ -11,6 +11,19 @@ extern "C" int tm_host_device_pointer(void* host, void** device) {
   return e == hipSuccess ? TM_OK : TM_ERR_HIP_BASE + (int)e;
 }
 
+extern "C" int tm_stream_capture_id(void* stream, uint64_t* id) {
+  if (id == nullptr) return TM_ERR_ARG;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long capture = 0;
+  const hipError_t e = hipStreamGetCaptureInfo((hipStream_t)stream, &status, &capture);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // not left for the next launch's check
+    return TM_ERR_HIP_BASE + (int)e;
+  }
+  *id = status == hipStreamCaptureStatusActive ? (uint64_t)capture + 1 : 0;
+  return TM_OK;
+}
+
 extern "C" const char* tm_status_string(int code) {
   switch (code) {
     case TM_OK:

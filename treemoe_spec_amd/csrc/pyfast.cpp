@@ -62,6 +62,15 @@ PyObject* py_attn_workspace(PyObject*, PyObject* args) {
   return Py_BuildValue("iL", rc, (long long)bytes);
 }
 
+// stream_capture_id(stream) -> (status, id)
+PyObject* py_stream_capture_id(PyObject*, PyObject* args) {
+  unsigned long long stream;
+  if (!PyArg_ParseTuple(args, "K", &stream)) return nullptr;
+  uint64_t id = 0;
+  const int rc = tm_stream_capture_id((void*)stream, &id);
+  return Py_BuildValue("iK", rc, (unsigned long long)id);
+}
+
 // tree_attention(...) -> status, the arguments of tm_tree_attention in order
 PyObject* py_tree_attention(PyObject*, PyObject* args) {
   unsigned long long q, kt, vt, kc, vc, table, scratch, mask, out, ws, stream;
@@ -83,6 +92,7 @@ PyObject* py_tree_attention(PyObject*, PyObject* args) {
 
 PyMethodDef kMethods[] = {
     {"attn_workspace", py_attn_workspace, METH_VARARGS, "tm_tree_attention_plan"},
+    {"stream_capture_id", py_stream_capture_id, METH_VARARGS, "tm_stream_capture_id"},
     {"tree_attention", py_tree_attention, METH_VARARGS, "tm_tree_attention"},
     {"argmax_walk", py_argmax_walk, METH_VARARGS, "tm_op4_argmax_walk"},
     {"kv_commit", py_kv_commit, METH_VARARGS, "tm_op4_kv_commit"},

@@ -19,6 +19,7 @@ from __future__ import annotations
 
 import ctypes
 import operator
+import threading
 import weakref
 
 import torch
@@ -38,13 +39,40 @@ except ImportError:  # not built: the ctypes binding is used
     _fast = None
 
 _mask_cache: dict = {}
+_CACHE_ENTRIES = 16
+
+
+def _capture_id(stream: int) -> int:
+    """0, or the identity of the graph capture under way on a raw stream (the
+    default stream, 0, cannot be captured)."""
+    if stream == 0:
+        return 0
+    if _fast is not None:
+        rc, cid = _fast.stream_capture_id(stream)
+        check(rc, "tm_stream_capture_id")
+        return cid
+    out = ctypes.c_uint64()
+    call("tm_stream_capture_id", stream, ctypes.byref(out))
+    return out.value
 
 
 def pack_tree_mask(tree_mask: torch.Tensor) -> torch.Tensor:
     """[N, N] bool device mask -> [N, ceil(N/64)] int64 bit words (bit j of row
-    i = tree_mask[i, j]); cached per live mask tensor and its version counter,
-    since the engine reuses one mask for every layer of a step."""
-    hit = _mask_cache.get(id(tree_mask))
+    i = tree_mask[i, j]), packed on the current stream of the mask's device.
+    Kept per live mask tensor and its version counter, since the engine reuses
+    one mask for every layer of a step."""
+    stream = _capi.stream_of(tree_mask.device)
+    return _packed_mask(tree_mask, stream, _capture_id(stream))
+
+
+def _packed_mask(tree_mask: torch.Tensor, stream: int, capture: int) -> torch.Tensor:
+    """pack_tree_mask for a raw stream and the capture under way on it.  The
+    words are used on the stream that packed them only, which orders both, and
+    inside a capture only where that capture packed them: words from before it
+    could be freed or become stale under the graph, and words packed inside it
+    hold nothing until a replay."""
+    key = (id(tree_mask), stream, capture)
+    hit = _mask_cache.get(key)
     if hit is not None and hit[0]() is tree_mask and hit[1] == tree_mask._version:
         return hit[2]
     n = tree_mask.shape[0]
@@ -52,11 +80,10 @@ def pack_tree_mask(tree_mask: torch.Tensor) -> torch.Tensor:
         raise ValueError("tree_mask must be [N, N] with unit stride along columns")
     m = tree_mask if tree_mask.dtype in (torch.bool, torch.uint8) else tree_mask.bool()
     bits = torch.empty(n, (n + 63) // 64, dtype=torch.int64, device=tree_mask.device)
-    call("tm_tree_mask_pack", ptr(m), n, m.stride(0), ptr(bits),
-         _capi.stream_of(tree_mask.device))
-    if len(_mask_cache) > 16:
+    call("tm_tree_mask_pack", ptr(m), n, m.stride(0), ptr(bits), stream)
+    if len(_mask_cache) > _CACHE_ENTRIES:
         _mask_cache.clear()
-    _mask_cache[id(tree_mask)] = (weakref.ref(tree_mask), tree_mask._version, bits)
+    _mask_cache[key] = (weakref.ref(tree_mask), tree_mask._version, bits)
     return bits
 
 
@@ -100,7 +127,9 @@ def tree_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv, layer:
     dev = q.device
     if scale is None:
         scale = hd ** -0.5
-    bits = pack_tree_mask(tree_mask)
+    stream = _capi.stream_of(dev)
+    capture = _capture_id(stream)
+    bits = _packed_mask(tree_mask, stream, capture)
     pages = scratch_pages_of(kv)
     page = kv.block_size
     if write_tree and len(pages) * page < n:
@@ -116,7 +145,7 @@ def tree_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv, layer:
         call("tm_tree_attention_plan", n, hq, kvh, hd, seq_len, page, chunk_keys,
              ctypes.byref(chunks), ctypes.byref(wbytes))
         nbytes = wbytes.value
-    ws = _workspace(nbytes, dev)
+    ws = _workspace(nbytes, dev, stream, capture)
     if out is None:
         out = torch.empty(n, hq * hd, dtype=torch.bfloat16, device=dev)
     elif out.shape != (n, hq * hd) or out.dtype != torch.bfloat16 or not out.is_contiguous():
@@ -127,7 +156,7 @@ def tree_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv, layer:
             page, table.data_ptr(), max(1, len(kv.block_table)), seq_len, scratch.data_ptr(),
             len(pages), 1 if write_tree else 0, bits.data_ptr(), n, hq, kvh, hd, float(scale),
             out.data_ptr(), hq * hd, chunk_keys, 0 if ws is None else ws.data_ptr(), nbytes,
-            _capi.stream_of(dev))
+            stream)
     if _fast is not None:
         check(_fast.tree_attention(*args), "tm_tree_attention")
     else:
@@ -138,14 +167,22 @@ def tree_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv, layer:
 _ws_cache: dict = {}
 
 
-def _workspace(nbytes: int, device) -> torch.Tensor | None:
-    """Chunk partials; one buffer per device, grown on demand (stream-ordered
-    reuse, like the reference's per-shape workspaces)."""
+def _workspace(nbytes: int, device, stream: int, capture: int) -> torch.Tensor | None:
+    """Chunk partials, written by a call's first launch and read by its second.
+    One buffer per (device, stream, calling thread), grown on demand: calls of
+    one thread on one stream reuse it in stream order, while calls of other
+    streams or threads may come between the two launches.  Under a graph capture
+    the buffer comes from the graph's pool and is not kept, so that no later
+    call can free or overwrite what the replays use."""
     if nbytes == 0:
         return None
-    key = torch.device(device)
+    if capture:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    key = (device, stream, threading.get_ident())
     buf = _ws_cache.get(key)
     if buf is None or buf.numel() < nbytes:
+        if buf is None and len(_ws_cache) >= _CACHE_ENTRIES:
+            _ws_cache.clear()
         buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
         _ws_cache[key] = buf
     return buf
