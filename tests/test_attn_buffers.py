@@ -73,3 +73,29 @@ def test_kept_workspaces_are_bounded(monkeypatch):
     for stream in range(1, 200):
         ta._workspace(16, CPU, stream, 0)
     assert len(ta._ws_cache) <= 32
+
+
+@pytest.mark.parametrize("foreign", [False, True])
+def test_block_table_keeps_its_device_buffer_as_the_sequence_grows(foreign):
+    """A captured graph holds the table's address: growing the sequence must fill the same
+    buffer, not put a new one in its place."""
+    from tests.ref_layout_cache import RefLayoutKVCache
+    from treemoe_spec_amd.kv_cache import MixtralConfig, PagedKVCache, device_tables_of
+
+    if foreign:
+        kv, page = RefLayoutKVCache(1, 2, 8, 12, device="cpu"), 64
+    else:
+        cfg = MixtralConfig(num_layers=1, num_kv_heads=2, head_dim=8, num_heads=2)
+        kv, page = PagedKVCache(cfg, 12, device="cpu", page_size=16, tree_size=8), 16
+    empty, scratch = device_tables_of(kv, "cpu")
+    address = empty.data_ptr()
+    for pages in (1, 3, 10):
+        kv._ensure_capacity(pages * page)
+        table, pages_again = device_tables_of(kv, "cpu")
+        assert table.tolist() == kv.block_table and table.data_ptr() == address
+        assert pages_again is scratch
+    # another mapping of the same length
+    kv.block_table.reverse()
+    if not foreign:
+        kv._dev_table_len = -1
+    assert device_tables_of(kv, "cpu")[0].tolist() == kv.block_table

@@ -40,6 +40,30 @@ class MixtralConfig:
         return 3 * self.intermediate_dim * self.hidden_dim * 2
 
 
+class _DeviceTables:
+    """int32 copies of a cache's block table and scratch pages on one device.  The
+    block table's buffer holds every page of the cache from the start and is
+    filled in place, so a captured graph, which holds its address, reads a valid
+    table however much the sequence has grown since."""
+
+    def __init__(self, device: torch.device, pages: int, scratch: list[int]):
+        self.device = device
+        self._buf = torch.zeros(max(1, pages), dtype=torch.int32, device=device)
+        self.scratch_list = list(scratch)
+        self.scratch = torch.tensor(scratch, dtype=torch.int32, device=device)
+        self.entries: list[int] | None = None
+        self.table = self._buf[:1]
+
+    def fill(self, block_table: list[int]) -> None:
+        n = len(block_table)
+        if n > self._buf.numel():  # a table that maps pages more than once
+            self._buf = torch.zeros(n, dtype=torch.int32, device=self.device)
+        if n:
+            self._buf[:n].copy_(torch.tensor(block_table, dtype=torch.int32))
+        self.entries = list(block_table)
+        self.table = self._buf[:max(1, n)]
+
+
 class PagedKVCache:
     def __init__(self, config, num_blocks: int, device: str = "cuda",
                  dtype: torch.dtype = torch.bfloat16, page_size: int = BLOCK_SIZE,
@@ -59,9 +83,8 @@ class PagedKVCache:
         self.tree_block = self.tree_pages[0]
         self.tree_size = tree_size
         self._free = list(range(num_blocks - 1, n_scratch - 1, -1))
-        self._dev_table: torch.Tensor | None = None
+        self._dev_tables: _DeviceTables | None = None
         self._dev_table_len = -1
-        self._dev_scratch: torch.Tensor | None = None
 
     # Positions map to flat slots of the [pages * page_size] axis:
     # slot = block_table[q // page_size] * page_size + q % page_size.  The
@@ -154,14 +177,14 @@ class PagedKVCache:
         device = torch.device(device)
         if device.type == "cuda" and device.index is None:
             device = torch.device("cuda", torch.cuda.current_device())
-        if self._dev_table is None or self._dev_table_len != len(self.block_table) \
-                or self._dev_table.device != device:
-            self._dev_table = torch.tensor(self.block_table or [0], dtype=torch.int32,
-                                           device=device)
+        t = self._dev_tables
+        if t is None or t.device != device:
+            t = self._dev_tables = _DeviceTables(device, self.k.shape[1], self.tree_pages)
+            self._dev_table_len = -1
+        if self._dev_table_len != len(self.block_table):
+            t.fill(self.block_table)
             self._dev_table_len = len(self.block_table)
-        if self._dev_scratch is None or self._dev_scratch.device != device:
-            self._dev_scratch = torch.tensor(self.tree_pages, dtype=torch.int32, device=device)
-        return self._dev_table, self._dev_scratch
+        return t.table, t.scratch
 
     def gather(self, layer: int, upto: int | None = None):
         """Contiguous [T, kv_heads, head_dim] K and V of positions 0..T-1
@@ -198,10 +221,10 @@ def scratch_pages_of(kv) -> list[int]:
     return list(pages) if pages is not None else [int(kv.tree_block)]
 
 
-# int32 device copies of the block table and scratch pages for caches without
-# ``device_tables`` (the reference's PagedKVCache), per cache object and
-# device, rebuilt when the host block table or scratch list changes.
-_table_cache: dict[tuple, tuple[list, list, torch.Tensor, torch.Tensor]] = {}
+# Tables of caches without ``device_tables`` (the reference's PagedKVCache): kept on
+# the cache object, or here for one that takes no attributes, and refilled when
+# the host block table or scratch list changes.
+_table_cache: dict[tuple, _DeviceTables] = {}
 
 
 def device_tables_of(kv, device) -> tuple[torch.Tensor, torch.Tensor]:
@@ -211,13 +234,16 @@ def device_tables_of(kv, device) -> tuple[torch.Tensor, torch.Tensor]:
     if hasattr(kv, "device_tables"):
         return kv.device_tables(device)
     pages = scratch_pages_of(kv)
-    key = (id(kv), torch.device(device))
-    hit = _table_cache.get(key)
-    if hit is not None and hit[0] == kv.block_table and hit[1] == pages:
-        return hit[2], hit[3]
-    table = torch.tensor(kv.block_table or [0], dtype=torch.int32, device=device)
-    scratch = torch.tensor(pages, dtype=torch.int32, device=device)
-    if len(_table_cache) > 16:
-        _table_cache.clear()
-    _table_cache[key] = (list(kv.block_table), pages, table, scratch)
-    return table, scratch
+    device = torch.device(device)
+    t = getattr(kv, "_tm_device_tables", None) or _table_cache.get((id(kv), device))
+    if t is None or t.device != device or t.scratch_list != pages:
+        t = _DeviceTables(device, kv.k.shape[1], pages)
+        try:
+            kv._tm_device_tables = t
+        except AttributeError:
+            if len(_table_cache) > 16:
+                _table_cache.clear()
+            _table_cache[(id(kv), device)] = t
+    if t.entries != kv.block_table:
+        t.fill(kv.block_table)
+    return t.table, t.scratch
