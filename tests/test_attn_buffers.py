@@ -99,3 +99,40 @@ def test_block_table_keeps_its_device_buffer_as_the_sequence_grows(foreign):
     if not foreign:
         kv._dev_table_len = -1
     assert device_tables_of(kv, "cpu")[0].tolist() == kv.block_table
+
+
+class _OnGpu(torch.Tensor):
+    """A CPU tensor that says it is on the GPU, to reach the launch arguments."""
+
+    is_cuda = property(lambda self: True)
+
+
+def test_layer_is_looked_up_in_both_caches(monkeypatch):
+    """K and V are addressed by their own layer counts: a V cache with fewer layers than K's is
+    refused where it ends, as indexing it is."""
+    from treemoe_spec_amd.kv_cache import MixtralConfig, PagedKVCache
+
+    cfg = MixtralConfig(num_layers=3, num_kv_heads=2, head_dim=128, num_heads=4)
+    kv = PagedKVCache(cfg, 4, device="cpu", page_size=16, tree_size=8)
+    kv._ensure_capacity(16)
+    kv.seq_len = 16
+    seen = {}
+    monkeypatch.setattr(ta, "_mask_cache", {})
+    monkeypatch.setattr(ta, "_fast", None)
+    monkeypatch.setattr(ta, "call", lambda name, *a: seen.update({name: a}))
+    monkeypatch.setattr(ta._capi, "stream_of", lambda dev: 0)
+    q = torch.zeros(4, 4, 128, dtype=torch.bfloat16).as_subclass(_OnGpu)
+    k = torch.zeros(4, 2, 128, dtype=torch.bfloat16)
+    att = lambda layer: ta.tree_attention(q, k, k, kv, layer, torch.eye(4, dtype=torch.bool))
+    for layer in (0, 2, -1, -3):
+        att(layer)
+        assert seen["tm_tree_attention"][5:7] == (kv.k[layer].data_ptr(), kv.v[layer].data_ptr())
+    for layer in (3, -4):
+        with pytest.raises(IndexError):
+            att(layer)
+    kv.v = kv.v[:2]
+    att(1)
+    assert seen["tm_tree_attention"][6] == kv.v[1].data_ptr()
+    for layer in (2, -3):
+        with pytest.raises(IndexError):
+            att(layer)
