@@ -103,3 +103,31 @@ def test_two_streams_have_their_own_partials():
     torch.cuda.synchronize()
     for j in range(2):
         assert all(torch.equal(o, want[j]) for o in got[j]), j
+
+
+def test_two_threads_on_one_stream():
+    """A call's two launches may have another thread's between them."""
+    import threading
+
+    from treemoe_spec_amd.kernels.tree_attention import tree_attention
+
+    print("attention from two threads", flush=True)
+    cases = [_on_gpu(33, 1500, 21), _on_gpu(33, 1500, 22)]
+    want = [tree_attention(q, k, v, kv, 0, mask, chunk_keys=64).clone()
+            for kv, q, k, v, mask in cases]
+    torch.cuda.synchronize()
+    got = [[], []]
+
+    def work(j):
+        kv, q, k, v, mask = cases[j]
+        for _ in range(60):
+            got[j].append(tree_attention(q, k, v, kv, 0, mask, chunk_keys=64))
+
+    threads = [threading.Thread(target=work, args=(j,)) for j in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for j in range(2):
+        assert len(got[j]) == 60 and all(torch.equal(o, want[j]) for o in got[j]), j

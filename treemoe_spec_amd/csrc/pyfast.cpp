@@ -1,7 +1,7 @@
 // _tmfast: a CPython binding of the per-step op4 greedy path and of the
-// per-layer tree attention of libtreemoe_amd.so.  The ctypes binding converts each argument through a
-// Python-level type object (~3.5 us per call of ~18 arguments on the GPU
-// host); this module parses them with PyArg_ParseTuple and calls the C ABI
+// per-layer tree attention of libtreemoe_amd.so.  The ctypes binding converts
+// each argument through a Python-level type object (~3.5 us per call of ~18
+// arguments on the GPU host); this module parses them with PyArg_ParseTuple and calls the C ABI
 // directly, so one greedy verify + KV commit costs one Python-to-C
 // transition.  It adds no semantics: every function here is a plain call of
 // the entry points declared in include/treemoe_amd.h.
@@ -82,11 +82,16 @@ PyObject* py_tree_attention(PyObject*, PyObject* args) {
                         &write_tree, &mask, &n, &hq, &kvh, &hd, &scale, &out, &os, &chunk, &ws,
                         &ws_bytes, &stream))
     return nullptr;
-  const int rc = tm_tree_attention(
+  int rc = 0;
+  // two launches, which wait when the stream's queue is full: the process's other
+  // threads run meanwhile, as in a ctypes call
+  Py_BEGIN_ALLOW_THREADS
+  rc = tm_tree_attention(
       (const void*)q, qs, (const void*)kt, (const void*)vt, ts, (void*)kc, (void*)vc, sp, ss, page,
       (const int32_t*)table, n_table, seq, (const int32_t*)scratch, n_scratch, write_tree,
       (const uint64_t*)mask, n, hq, kvh, hd, scale, (void*)out, os, chunk, (void*)ws, ws_bytes,
       (void*)stream);
+  Py_END_ALLOW_THREADS
   return PyLong_FromLong(rc);
 }
 
