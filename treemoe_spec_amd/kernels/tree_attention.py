@@ -87,14 +87,6 @@ def _packed_mask(tree_mask: torch.Tensor, stream: int, capture: int) -> torch.Te
     return bits
 
 
-def _layer_address(cache: torch.Tensor, layer: int) -> int:
-    """Device address of cache[layer], refused as the indexing refuses it."""
-    layers = cache.shape[0]
-    if not -layers <= layer < layers:
-        raise IndexError(f"layer {layer} is out of range for a cache of {layers} layers")
-    return cache.data_ptr() + cache.element_size() * cache.stride(0) * (layer % layers)
-
-
 def tree_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv, layer: int,
                    tree_mask: torch.Tensor, scale: float | None = None,
                    out: torch.Tensor | None = None, write_tree: bool = True,
@@ -126,14 +118,17 @@ def tree_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv, layer:
     if kc.dtype != torch.bfloat16 or cshape[3] != kvh or cshape[4] != hd:
         raise ValueError("cache layout must be [L, pages, page, kv_heads, head_dim] bf16")
     layer = operator.index(layer)
-    p_kc, p_vc = _layer_address(kc, layer), _layer_address(vc, layer)
+    layers, vlayers = cshape[0], vc.shape[0]  # refused where indexing either refuses it
+    if not (-layers <= layer < layers and -vlayers <= layer < vlayers):
+        raise IndexError(f"layer {layer} is out of range for a cache of "
+                         f"{min(layers, vlayers)} layers")
     if tuple(tree_mask.shape) != (n, n):
         raise ValueError("tree_mask must be [N, N]")
     dev = q.device
     if scale is None:
         scale = hd ** -0.5
     stream = _capi.stream_of(dev)
-    capture = _capture_id(stream)
+    capture = _capture_id(stream) if stream else 0
     bits = _packed_mask(tree_mask, stream, capture)
     pages = scratch_pages_of(kv)
     page = kv.block_size
@@ -155,8 +150,10 @@ def tree_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv, layer:
         out = torch.empty(n, hq * hd, dtype=torch.bfloat16, device=dev)
     elif out.shape != (n, hq * hd) or out.dtype != torch.bfloat16 or not out.is_contiguous():
         raise ValueError("out must be a contiguous [N, Hq * hd] bf16 tensor")
-    cs = kc.stride()
-    args = (q.data_ptr(), qs[0], k.data_ptr(), v.data_ptr(), ks[0], p_kc, p_vc, cs[1], cs[2],
+    cs, vcs = kc.stride(), vc.stride()
+    args = (q.data_ptr(), qs[0], k.data_ptr(), v.data_ptr(), ks[0],
+            kc.data_ptr() + 2 * cs[0] * (layer % layers),
+            vc.data_ptr() + 2 * vcs[0] * (layer % vlayers), cs[1], cs[2],
             page, table.data_ptr(), max(1, len(kv.block_table)), seq_len, scratch.data_ptr(),
             len(pages), 1 if write_tree else 0, bits.data_ptr(), n, hq, kvh, hd, float(scale),
             out.data_ptr(), hq * hd, chunk_keys, 0 if ws is None else ws.data_ptr(), nbytes,

@@ -41,27 +41,31 @@ class MixtralConfig:
 
 
 class _DeviceTables:
-    """int32 copies of a cache's block table and scratch pages on one device.  The
-    block table's buffer holds every page of the cache from the start and is
-    filled in place, so a captured graph, which holds its address, reads a valid
-    table however much the sequence has grown since."""
+    """int32 copies of a cache's scratch page list and block table on one device, in
+    one buffer with room for every page of the cache.  The block table is filled
+    in place, so a captured graph, which holds its address, reads a valid table
+    however much the sequence has grown since."""
 
     def __init__(self, device: torch.device, pages: int, scratch: list[int]):
         self.device = device
-        self._buf = torch.zeros(max(1, pages), dtype=torch.int32, device=device)
         self.scratch_list = list(scratch)
-        self.scratch = torch.tensor(scratch, dtype=torch.int32, device=device)
         self.entries: list[int] | None = None
-        self.table = self._buf[:1]
+        self._pages = pages
+        self._buf: torch.Tensor | None = None
 
     def fill(self, block_table: list[int]) -> None:
-        n = len(block_table)
-        if n > self._buf.numel():  # a table that maps pages more than once
-            self._buf = torch.zeros(n, dtype=torch.int32, device=self.device)
-        if n:
-            self._buf[:n].copy_(torch.tensor(block_table, dtype=torch.int32))
+        s, n = len(self.scratch_list), len(block_table)
+        host, at = block_table, s
+        if self._buf is None or self._buf.numel() < s + n:
+            # (a table longer than the cache maps pages more than once)
+            self._buf = torch.empty(s + max(1, self._pages, n), dtype=torch.int32,
+                                    device=self.device)
+            self.scratch = self._buf[:s]
+            host, at = self.scratch_list + block_table, 0
+        if host:
+            self._buf[at:s + n].copy_(torch.tensor(host, dtype=torch.int32))
         self.entries = list(block_table)
-        self.table = self._buf[:max(1, n)]
+        self.table = self._buf[s:s + max(1, n)]
 
 
 class PagedKVCache:
