@@ -179,9 +179,9 @@ int tm_op1_combine(const float* y, const int32_t* slot_pos, void* out,
 
 /*
  * Gate/up projection + SwiGLU for many rows per expert (prefill / batched
- * trees), MFMA-tiled over 128 sorted rows x (128 w1 + the same 128 w3) weight
- * rows; 256 rows when 2T >= 384 E, and 64 rows x (64 + 64) weight rows when
- * 2T <= 16 max_tiles (few rows per active expert).  Same maths as
+ * trees), MFMA-tiled over 256 or 128 sorted rows x (128 w1 + the same 128 w3)
+ * weight rows, or 64 rows x (64 + 64) weight rows; tm_op1_prefill_tiles tells
+ * which.  Same maths as
  * tm_op1_gemm1 and the reference `_moe_gemm1_kernel`
  * (treemoe/kernels/op1_tree_moe.py:300-383), but h is written ROW-MAJOR:
  *   h[p, n] = bf16( silu(x[sorted_slots[p] / 2] . w1[e, n]) * (... . w3[e, n]) )
@@ -195,6 +195,16 @@ int tm_op1_prefill_gemm1(const void* x, const void* w1, const void* w3, void* h,
                          const int32_t* sorted_slots, const int32_t* expert_offsets,
                          const int32_t* tiles, int64_t max_tiles, int64_t T, int64_t H,
                          int64_t I, int64_t E, int dtype, void* stream);
+
+/*
+ * Rows of the M-tiles that tm_op1_prefill_gemm1 (*gate_up) and
+ * tm_op1_prefill_gemm2 (*down) take for these sizes: 256 where 2T >= 112 E and
+ * half as many, twice as tall jobs fill the GPU in less time, 64 at few rows per
+ * expert, else 128.  The bits of h and y do not depend on it.  For naming
+ * kernels in measurements; no reference counterpart.
+ */
+int tm_op1_prefill_tiles(int64_t max_tiles, int64_t split, int64_t T, int64_t H,
+                         int64_t I, int64_t E, int64_t* gate_up, int64_t* down);
 
 /*
  * tm_op1_route_bucket and tm_op1_prefill_gemm1 in ONE launch, for few tokens:
@@ -220,8 +230,8 @@ int tm_op1_prefill_gemm1_routed(const void* x, const void* w1, const void* w3, v
                                 int32_t* slot_pos, int32_t* tiles, int dtype, void* stream);
 
 /*
- * Down projection for many rows per expert, MFMA-tiled over 128 rows x 256
- * output columns; the prefill counterpart of tm_op1_gemm2 (reference
+ * Down projection for many rows per expert, MFMA-tiled over 256 or 128 rows x
+ * 256 output columns, or 64 rows x 128 (tm_op1_prefill_tiles); the prefill counterpart of tm_op1_gemm2 (reference
  * `_moe_gemm2_det_kernel`, treemoe/kernels/op1_tree_moe.py:447-509):
  *   y[s, p, n] = gates_flat[sorted_slots[p]] * sum_{k in segment s} h[p, k] w2[e, n, k]
  * with h row-major [2T, I] from tm_op1_prefill_gemm1 and y [split, 2T, H] fp32

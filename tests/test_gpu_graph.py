@@ -60,7 +60,7 @@ def _replays_match(g, out, want, eager_between):
     ("tiled", 64, 4),
     ("tiled_bucket", 64, 4),   # router + bucketing launches, then the tiled pair
     ("stream", 64, 8),         # the weight-streaming pair
-    ("tiled", 512, 8),         # many rows per expert: the 256-row ping-pong tiles
+    ("tiled", 512, 8),         # many rows per expert: the 256-row tiles
 ])
 def test_op1_graph_replays_equal_eager(path, t, budget, monkeypatch):
     _say(f"graph capture op1 path={path} t={t} B={budget}")
@@ -69,7 +69,7 @@ def test_op1_graph_replays_equal_eager(path, t, budget, monkeypatch):
     monkeypatch.setattr(m, "TILED_MIN_ROWS_WIDE", 1 << 30 if path == "stream" else 1)
     if path == "tiled_bucket":
         monkeypatch.setattr(m, "SELF_ROUTED_MAX_TOKENS", 0)
-    e, h, i = (8, 512, 1024) if t <= 64 else (2, 512, 1024)
+    e, h, i = (8, 512, 1024) if t <= 64 else (2, 512, 6144)
     g = torch.Generator().manual_seed(900 + t + budget)
     x, w1, w2, w3, router, accept = make_moe_inputs(t, e, h, i, g, dtype=torch.bfloat16)
     dev = [a.cuda() for a in (x, w1, w2, w3, router, accept)]

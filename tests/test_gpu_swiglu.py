@@ -11,6 +11,8 @@ that of a log2(e) rounded to fp32, at most |a| 2^-24 relative, plus one unit
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -18,19 +20,21 @@ pytestmark = pytest.mark.gpu
 
 # e^-a overflows fp32 below this: silu is then -0
 OVERFLOW = -88.72
-TILES = [("256 rows", 2, 14), ("128 rows", 8, 14), ("64 rows", 8, 52)]
+# rows of the tile, experts, tile-list length, hidden, intermediate size
+TILES = [(256, 2, 14, 256, 6144), (128, 8, 14, 64, 256), (64, 8, 52, 64, 256)]
 
 
-def _gate_up(tile, experts, max_tiles, a, c, b, dtype):
+def _gate_up(tile, experts, max_tiles, h, a, c, b, dtype):
     """(h, a, c per row): experts 0 and 1 hold every token, the others none."""
     from treemoe_spec_amd import _capi
 
     dev = torch.device("cuda")
-    t, h, i = a.numel(), 64, b.numel()
+    t, i = a.numel(), b.numel()
     rows = 2 * t
-    # the rule of tm_op1_prefill_gemm1: 256 rows, else 64 rows, else 128
-    assert tile == ("256 rows" if rows >= 112 * experts else
-                    "64 rows" if rows <= 16 * max_tiles else "128 rows")
+    taken = ctypes.c_int64()
+    _capi.call("tm_op1_prefill_tiles", max_tiles, 1, t, h, i, experts, ctypes.byref(taken),
+               ctypes.byref(ctypes.c_int64()))
+    assert taken.value == tile
     x = torch.zeros(t, h)
     x[:, 0], x[:, 1] = a, c
     w1, w3 = torch.zeros(experts, i, h), torch.zeros(experts, i, h)
@@ -52,14 +56,14 @@ def _gate_up(tile, experts, max_tiles, a, c, b, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("tile,experts,max_tiles", TILES)
-def test_swiglu_range_matches_float64(tile, experts, max_tiles, dtype):
-    print(f"swiglu {tile} {dtype}", flush=True)
+@pytest.mark.parametrize("tile,experts,max_tiles,hidden,inter", TILES)
+def test_swiglu_range_matches_float64(tile, experts, max_tiles, hidden, inter, dtype):
+    print(f"swiglu {tile} rows {dtype}", flush=True)
     a = torch.cat([torch.arange(-100.0, 100.25, 0.5), torch.zeros(1)])   # exact in 16 bits
     # b over the powers of two that the type holds
     powers = [-60, -10, 0, 8, 30, 60, 90, 120] if dtype == torch.bfloat16 else [-8, -4, -1, 0, 1, 4]
-    b = torch.tensor([2.0 ** powers[n % len(powers)] for n in range(256)])
-    h, av, _ = _gate_up(tile, experts, max_tiles, a, torch.ones_like(a), b, dtype)
+    b = torch.tensor([2.0 ** powers[n % len(powers)] for n in range(inter)])
+    h, av, _ = _gate_up(tile, experts, max_tiles, hidden, a, torch.ones_like(a), b, dtype)
     out = h.double()
     ref = av * torch.sigmoid(av) * b.double()
     info = torch.finfo(dtype)
@@ -71,16 +75,16 @@ def test_swiglu_range_matches_float64(tile, experts, max_tiles, dtype):
     assert not bad.any(), (av.expand_as(ref)[bad][:4], out[bad][:4], ref[bad][:4])
 
 
-@pytest.mark.parametrize("tile,experts,max_tiles", TILES)
-def test_fp16_h_is_rounded_once(tile, experts, max_tiles):
+@pytest.mark.parametrize("tile,experts,max_tiles,hidden,inter", TILES)
+def test_fp16_h_is_rounded_once(tile, experts, max_tiles, hidden, inter):
     """fp16 h where silu(a) = a exactly (e^-a below half a unit of 1) and b is a product of two
     11-bit values: the 33-bit product a b rounded once to fp16, not to fp32 first."""
-    print(f"fp16 rounding {tile}", flush=True)
+    print(f"fp16 rounding {tile} rows", flush=True)
     g = torch.Generator().manual_seed(5)
     a = (18.0 + 40.0 * torch.rand(402, generator=g)).half().float()
     c = (1.0 + torch.rand(402, generator=g)).half().float()
-    b = (1.0 + torch.rand(256, generator=g)).half().float()
-    h, av, cv = _gate_up(tile, experts, max_tiles, a, c, b, torch.float16)
+    b = (1.0 + torch.rand(inter, generator=g)).half().float()
+    h, av, cv = _gate_up(tile, experts, max_tiles, hidden, a, c, b, torch.float16)
     exact = (av * cv * b.double()).numpy()
     once = torch.from_numpy(exact.astype("float16"))
     twice = torch.from_numpy(exact.astype("float32").astype("float16"))

@@ -9,6 +9,8 @@ magnitudes); h is then rounded to 16 bits (2^-9 relative in bf16), y is not.
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -27,17 +29,26 @@ def _layout(dev, g):
     return offsets, slots, as_dev(offsets), slots.to(dev), as_dev(tiles), len(tiles)
 
 
-@pytest.mark.parametrize("steps", [1, 4, 5, 6, 7, 8, 9])
+def _tiles(max_tiles, split, t, h, i, e):
+    from treemoe_spec_amd import _capi
+
+    out = (ctypes.c_int64 * 2)()
+    _capi.call("tm_op1_prefill_tiles", max_tiles, split, t, h, i, e, ctypes.byref(out),
+               ctypes.byref(out, 8))
+    return tuple(out)
+
+
+@pytest.mark.parametrize("steps", [4, 5, 6, 7, 8, 9])
 def test_tile256_gemms_match_float64(steps):
     from treemoe_spec_amd import _capi
 
     dev = torch.device("cuda")
     g = torch.Generator().manual_seed(steps)
     e, rows = len(COUNTS), sum(COUNTS)
-    t, h, i = rows // 2, 64 * steps, 256
-    assert rows % 2 == 0 and rows >= 112 * e      # the 256-row tile's rule
+    t, h, i = rows // 2, 64 * steps, 2048
     print(f"tile256 steps={steps}", flush=True)
     offsets, slots, off_d, slots_d, tiles_d, nt = _layout(dev, g)
+    assert rows % 2 == 0 and _tiles(nt, 1, t, h, i, e)[0] == 256
     draw = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
     x, w1, w3 = draw(t, h), draw(e, i, h) * 0.1, draw(e, i, h) * 0.1
     xd, w1d, w3d = x.to(dev), w1.to(dev), w3.to(dev)
@@ -57,8 +68,9 @@ def test_tile256_gemms_match_float64(steps):
         tol = 2.0 ** -8 * ref.abs() + 1e-5 * (1.0 + a.abs()) * (1.0 + b.abs())
         assert torch.all((out[r] - ref).abs() <= tol), (steps, COUNTS[k])
 
-    # down: K = 64 * steps per segment, two segments, H = 256
-    ki, n = 128 * steps, 256
+    # down: K = 64 * steps per segment, two segments
+    ki, n = 128 * steps, 2048
+    assert _tiles(nt, 2, t, n, ki, e)[1] == 256
     hm, w2 = draw(rows, ki), draw(e, n, ki) * 0.1
     gates = torch.rand(rows, generator=g)
     hmd, w2d, gd = hm.to(dev), w2.to(dev), gates.to(dev)
@@ -91,7 +103,7 @@ def test_narrow_down_tile_matches_float64(counts):
     for k, c in enumerate(counts):
         tiles += [[k, offsets[k] + r0, min(64, c - r0), 0] for r0 in range(0, c, 64)]
         offsets.append(offsets[-1] + c)
-    assert 2 * t <= 64 * e and len(tiles) * (n // 256) * 4 < 256    # the rule
+    assert _tiles(len(tiles), 4, t, n, ki, e)[1] == 64
     print(f"narrow down {counts}", flush=True)
     draw = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
     hm, w2, gates = draw(rows, ki), draw(e, n, ki) * 0.1, torch.rand(rows, generator=g)

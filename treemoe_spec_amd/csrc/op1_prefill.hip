@@ -18,7 +18,7 @@
 //
 // Three tile configurations:
 //   Tile256  256 rows x 256 weight rows on 4 waves, one per SIMD, hand-
-//            pipelined (PipeLoop): where the experts average 112 rows or more;
+//            pipelined (PipeLoop): many rows per expert and enough jobs (use_tile256);
 //   Tile128  128 x 256 on 8 waves, three 48 KB stages;
 //   TileDec  64 x 128 on 4 waves, three 24 KB stages, so two workgroups share
 //            a CU: gate/up when the tile list leaves at most 16 rows per entry,
@@ -41,6 +41,7 @@
 #pragma clang fp contract(off)
 
 #include <algorithm>
+#include <cmath>
 
 #include "op1_bucket.h"
 #include "tm_common.h"
@@ -1045,8 +1046,67 @@ tm_prefill_gemm2_kernel(const uint16_t* __restrict__ h, const uint16_t* __restri
 
 bool aligned16(const void* p) { return ((uintptr_t)p % 16) == 0; }
 
-// The experts average 112 rows or more: Tile256 (see tm_op1_prefill_gemm1).
-bool many_rows(int64_t T, int64_t E) { return 2 * T >= 112 * E; }
+// M-tiles of BM rows that `active` experts averaging `rows` rows take, their loads
+// taken as spread evenly over +-20 % of the average.
+double expected_mtiles(double active, double rows, int BM) {
+  const double lo = 0.8 * rows, hi = 1.2 * rows;
+  int64_t k = (int64_t)(lo / BM) + 1;
+  double n = (double)k;
+  for (; (double)(k * BM) < hi; ++k) n += (hi - (double)(k * BM)) / (hi - lo);
+  return active * n;
+}
+
+// Tile256 for a GEMM of `ncol` column jobs (256 weight rows each) whose jobs run
+// over K: where the experts average 112 rows or more, and its jobs, half as many
+// as Tile128's, still come out ahead in rounds over the CUs.  An XCD runs its
+// cpx columns of every M-tile on its 32 CUs (a last round counts in full once it
+// is likely to have a sixth of the CUs' jobs); a Tile256 round takes 1.3 + 150 / K
+// Tile128 rounds (the prologue and epilogue weigh more at a short K).  From 112
+// rows on an expert often has more rows than a 128-row tile holds, and its
+// weights pass through LDS twice.  Tile128 against Tile256, same box, us:
+//   H = 4096, I = 14336, E = 8   T = 448 gate/up 343 / 366, down 253 / 168;
+//     T = 517 418 / 370, 241 / 163; T = 2048 1028 / 890, 538 / 484
+//   H = 4096, I = 1792, E = 8    T = 700 70 / 80, 43 / 48; T = 1200 114 / 89, 66 / 51
+//   H = 1024, I = 3584, E = 8    T = 700 41 / 40, 25 / 33; T = 1200 55 / 64, 39 / 35
+//   H = 512, I = 2048, E = 8     T = 700 18 / 27, 17 / 24; T = 3000 51 / 48, 33 / 28
+// Over 348 layers of H = 256 .. 4096, E = 2 .. 64, T = 112 .. 6000, the tile it picks
+// is 2 % behind the better of the two in the mean, the 256-row tile everywhere
+// 12 %.
+bool use_tile256(int64_t T, int64_t E, int64_t max_tiles, int64_t ncol, int64_t K) {
+  if (2 * T < 112 * E) return false;
+  // the routed experts, from the tile list's bound: a + (2T - a) / 64 tiles
+  int64_t active = 1;
+  while (active < E && active + (2 * T - active) / TM_GEMM_TILE_M < max_tiles) ++active;
+  const double rows = 2.0 * (double)T / (double)active;
+  const double cpx = (double)((ncol + kXcds - 1) / kXcds);
+  const auto rounds = [&](int BM) {
+    const double r = expected_mtiles((double)active, rows, BM) * cpx / (kCUs / kXcds);
+    return std::floor(r) + std::min(1.0, 6.0 * (r - std::floor(r)));
+  };
+  return (1.3 + 150.0 / (double)K) * rounds(256) <= rounds(128);
+}
+
+// Rows of the gate/up tile.  TileDec when the tile list leaves at most 16 rows per
+// entry (2T <= 16 max_tiles: few rows per active expert, e.g. 64 tree tokens over
+// 8 experts): half the weight rows per workgroup and two workgroups per CU
+// stream the weights faster there (config 2 gate/up 302 -> 289 us same-box).
+int gate_up_rows(int64_t max_tiles, int64_t T, int64_t H, int64_t I, int64_t E) {
+  if (use_tile256(T, E, max_tiles, I / (Tile256::PBN / 2), H)) return 256;
+  return 2 * T <= 16 * max_tiles ? 64 : 128;
+}
+
+// Rows of the down tile.  TileDec (twice the column jobs, two workgroups per CU)
+// where the 128-row tile's jobs leave CUs without one and few experts exceed its
+// 64 rows.  Down + combine on Tile128 against TileDec, four K segments, E = 8,
+// I = 3584: H = 1024 (at most 144 jobs) T = 16 18.2 against 14.6 us, T = 64 18.9 /
+// 15.1, T = 64 budget 4 19.8 / 14.1, T = 200 23.3 / 18.6; where the jobs fill the
+// CUs, H = 4096, I = 14336, T = 64 budget 4 79.7 / 84.0.
+int down_rows(int64_t max_tiles, int64_t split, int64_t T, int64_t H, int64_t I, int64_t E) {
+  const int64_t ncol = H / Tile128::PBN * split;
+  if (use_tile256(T, E, max_tiles, ncol, I / split)) return 256;
+  const int64_t mt128 = std::min<int64_t>(max_tiles, mtile_bound<Tile128>(2 * T, E));
+  return 2 * T <= 64 * E && mt128 * ncol < kCUs ? 64 : 128;
+}
 
 // The gate/up launch with tile C: jobs for the M-tile bound (the tile list's
 // length, capped by what 2T rows in E experts can take).
@@ -1101,27 +1161,16 @@ extern "C" int tm_op1_prefill_gemm1(const void* x, const void* w1, const void* w
   if (I * H * 2 >= (int64_t)kOOR || T * H * 2 >= (int64_t)kOOR || 2 * T * I * 2 >= (int64_t)kOOR)
     return TM_ERR_SHAPE;
   if (!aligned16(x) || !aligned16(w1) || !aligned16(w3) || !aligned16(h)) return TM_ERR_ALIGN;
-  // 256-row tiles where the experts average 112 rows or more: from there an
-  // expert often has more rows than a 128-row tile holds, and its weights would
-  // pass through LDS twice.  H = 4096, I = 14336, E = 8, gate/up + down on
-  // Tile128 against Tile256: T = 400 490 against 502 us, T = 430 496 against
-  // 503, T = 460 (115 rows) 580 against 505, T = 517 680 against 519, T = 1030
-  // 918 against 896.  TileDec when
-  // the tile list leaves at most 16 rows per entry (2T <= 16 max_tiles: few
-  // rows per active expert, e.g. 64 tree tokens over 8 experts): half the
-  // weight rows per workgroup and two workgroups per CU stream the weights
-  // faster there (config 2 gate/up 302 -> 289 us same-box).
-  const bool big = many_rows(T, E);
-  const bool dec = !big && 2 * T <= 16 * max_tiles;
+  const int tile = gate_up_rows(max_tiles, T, H, I, E);
   const hipStream_t st = (hipStream_t)stream;
   const bool f16 = dtype == TM_DTYPE_F16;
   int rc;
-  if (big) {
+  if (tile == 256) {
     rc = f16 ? launch_gemm1<Tile256, TM_DTYPE_F16>(x, w1, w3, h, sorted_slots, expert_offsets,
                                                    tiles, max_tiles, T, H, I, E, st)
              : launch_gemm1<Tile256, TM_DTYPE_BF16>(x, w1, w3, h, sorted_slots, expert_offsets,
                                                     tiles, max_tiles, T, H, I, E, st);
-  } else if (dec) {
+  } else if (tile == 64) {
     rc = f16 ? launch_gemm1<TileDec, TM_DTYPE_F16>(x, w1, w3, h, sorted_slots, expert_offsets,
                                                    tiles, max_tiles, T, H, I, E, st)
              : launch_gemm1<TileDec, TM_DTYPE_BF16>(x, w1, w3, h, sorted_slots, expert_offsets,
@@ -1134,6 +1183,17 @@ extern "C" int tm_op1_prefill_gemm1(const void* x, const void* w1, const void* w
   }
   if (rc) return rc;
   TM_HIP_CHECK_LAUNCH();
+  return TM_OK;
+}
+
+extern "C" int tm_op1_prefill_tiles(int64_t max_tiles, int64_t split, int64_t T, int64_t H,
+                                    int64_t I, int64_t E, int64_t* gate_up, int64_t* down) {
+  if (T < 1 || T > TM_MAX_TOKENS || E < 2 || E > TM_MAX_EXPERTS || max_tiles < 1 || split < 1 ||
+      H < 1 || I < split)
+    return TM_ERR_SHAPE;
+  if (gate_up == nullptr || down == nullptr) return TM_ERR_ARG;
+  *gate_up = gate_up_rows(max_tiles, T, H, I, E);
+  *down = down_rows(max_tiles, split, T, H, I, E);
   return TM_OK;
 }
 
@@ -1232,22 +1292,15 @@ extern "C" int tm_op1_prefill_gemm2(const void* h, const void* w2, float* y,
   if (klen < C::PBK || (klen % C::PBK) != 0 || H < C::PBN || (H % C::PBN) != 0) return TM_ERR_SHAPE;
   if (H * I * 2 >= (int64_t)kOOR || 2 * T * I * 2 >= (int64_t)kOOR) return TM_ERR_SHAPE;
   if (!aligned16(h) || !aligned16(w2) || !aligned16(y)) return TM_ERR_ALIGN;
-  // many_rows: the gate/up rule.  TileDec (twice the column jobs, two workgroups
-  // per CU) where the 128-row tile's jobs leave CUs without one and few experts
-  // exceed its 64 rows.  Down + combine on Tile128 against TileDec, four K
-  // segments, E = 8, I = 3584: H = 1024 (at most 144 jobs) T = 16 18.2 against
-  // 14.6 us, T = 64 18.9 / 15.1, T = 64 budget 4 19.8 / 14.1, T = 200 23.3 / 18.6;
-  // where the jobs fill the CUs, H = 4096, I = 14336, T = 64 budget 4 79.7 / 84.0.
-  const int64_t mt128 = std::min<int64_t>(max_tiles, mtile_bound<Tile128>(2 * T, E));
-  const bool dec = 2 * T <= 64 * E && mt128 * (H / C::PBN) * split < kCUs;
+  const int tile = down_rows(max_tiles, split, T, H, I, E);
+  const hipStream_t st = (hipStream_t)stream;
   const int rc =
-      many_rows(T, E)
-          ? launch_gemm2<Tile256>(h, w2, y, gates_flat, sorted_slots, expert_offsets, tiles,
-                                  max_tiles, split, T, H, I, E, dtype, (hipStream_t)stream)
-      : dec ? launch_gemm2<TileDec>(h, w2, y, gates_flat, sorted_slots, expert_offsets, tiles,
-                                    max_tiles, split, T, H, I, E, dtype, (hipStream_t)stream)
-            : launch_gemm2<Tile128>(h, w2, y, gates_flat, sorted_slots, expert_offsets, tiles,
-                                    max_tiles, split, T, H, I, E, dtype, (hipStream_t)stream);
+      tile == 256  ? launch_gemm2<Tile256>(h, w2, y, gates_flat, sorted_slots, expert_offsets,
+                                           tiles, max_tiles, split, T, H, I, E, dtype, st)
+      : tile == 64 ? launch_gemm2<TileDec>(h, w2, y, gates_flat, sorted_slots, expert_offsets,
+                                           tiles, max_tiles, split, T, H, I, E, dtype, st)
+                   : launch_gemm2<Tile128>(h, w2, y, gates_flat, sorted_slots, expert_offsets,
+                                           tiles, max_tiles, split, T, H, I, E, dtype, st);
   if (rc) return rc;
   TM_HIP_CHECK_LAUNCH();
   return TM_OK;
