@@ -34,3 +34,18 @@ def test_layer_out_of_range_is_refused():
     kv, q, k, v, mask = _case(4, 8, 2, 20, 16, 3)
     with pytest.raises(IndexError):
         tree_attention(q.cuda(), k.cuda(), v.cuda(), kv, 2, mask.cuda())
+
+
+@pytest.mark.parametrize("n,hq,kvh", [(72, 32, 8), (73, 32, 8), (80, 32, 8), (81, 32, 8),
+                                      (97, 32, 32), (33, 64, 64)])
+def test_combine_with_many_units(n, hq, kvh):
+    """On both sides of the unit count (KV heads x 32-row groups x 16) from which one wave merges
+    a unit's chunks; the last row group partly empty."""
+    from treemoe_spec_amd.kernels.tree_attention import tree_attention
+
+    for seq_len in (64, 190, 1030):
+        print(f"attention combine n={n} hq={hq} kvh={kvh} seq={seq_len}", flush=True)
+        kv, q, k, v, mask = _case(n, hq, kvh, seq_len, 16, 5 * n + seq_len)
+        want = _oracle(kv, q, k, v, mask, 1)
+        _check(tree_attention(q.cuda(), k.cuda(), v.cuda(), kv, 1, mask.cuda(), chunk_keys=64),
+               want)

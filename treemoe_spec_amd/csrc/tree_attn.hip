@@ -447,21 +447,26 @@ __global__ void __launch_bounds__(kThreads, 2) tm_tree_attn_kernel(AttnParams p)
   }
 }
 
-// One workgroup per (KV head, row block, 32-row group, 4-value group): its four
-// waves merge the chunks c with c % 4 = wave, in chunk order with a running
-// maximum,
+// Merges the chunks of a unit (KV head, row block, 32-row group, 4-value group) in
+// chunk order with a running maximum,
 //   w_c = l_c 2^(m_c - M),  O = sum_c w_c O_c / sum_c w_c,
-// keeping the running sums against the running maximum, and the first wave
-// merges the four in wave order.  The kernel is bound by the latency of its
-// loads: one wave over all chunks waited for four at a time, one after the
-// other.  Whole call, 32 query over 8 KV heads, together with the waves without
-// rows above: one node over 1000 / 3000 / 7777 positions 11.9 / 16.0 / 19.0 ->
-// 9.5 / 11.8 / 15.3 us, 27 nodes over 333 11.5 -> 10.5, 64 over 4096 20.0 -> 20.0.
+// keeping the running sums against the running maximum.
+// W = 4: a workgroup per unit; wave w takes the chunks c with c % 4 = w and the
+// first wave merges the four in wave order.  With few units the kernel is bound
+// by the latency of its loads: one wave over all chunks waited for four at a
+// time, one after the other.  Whole call, 32 query over 8 KV heads, together with
+// the waves without rows above: one node over 1000 / 3000 / 7777 positions 11.9 /
+// 16.0 / 19.0 -> 9.5 / 11.8 / 15.3 us, 27 nodes over 333 11.5 -> 10.5, 64 over
+// 4096 20.0 -> 20.0.
+// W = 1: a wave per unit, where the units alone fill the chip (combine_waves).
+template <int W>
 __global__ void __launch_bounds__(kThreads) tm_tree_attn_combine_kernel(AttnParams p) {
-  __shared__ float s_o[3][6][64];
+  static_assert(W == 1 || W == 4, "waves per unit");
+  __shared__ float s_o[W == 4 ? 3 : 1][6][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int grp = (int)(blockIdx.x & 15);     // (ht, gq) = (grp / 4, grp % 4)
-  const int kw = (int)(blockIdx.x >> 4);      // (kvhead * row_blocks + rb) * 4 + 32-row group
+  const int unit = W == 4 ? (int)blockIdx.x : (int)blockIdx.x * 4 + wave;
+  const int grp = unit & 15;                  // (ht, gq) = (grp / 4, grp % 4)
+  const int kw = unit >> 4;                   // (kvhead * row_blocks + rb) * 4 + 32-row group
   const int rg = kw & 3, kr = kw >> 2;
   const int rb = kr % p.row_blocks, kvhead = kr / p.row_blocks;
   if (rb * kRows + rg * 32 >= p.rows) return;
@@ -469,7 +474,7 @@ __global__ void __launch_bounds__(kThreads) tm_tree_attn_combine_kernel(AttnPara
   float m_run = -INFINITY, w_sum = 0.0f;
   f32x4_t o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
-  for (int c = wave; c < p.chunks; c += 4) {
+  for (int c = W == 4 ? wave : 0; c < p.chunks; c += W) {
     const int64_t slot = ((int64_t)kr * p.chunks + c) * 4 + rg;
     const f32x2_t st = *reinterpret_cast<const f32x2_t*>(p.stats + slot * kStatFloats + c32 * 2);
     const f16x4_t hc = *reinterpret_cast<const f16x4_t*>(
@@ -485,26 +490,29 @@ __global__ void __launch_bounds__(kThreads) tm_tree_attn_combine_kernel(AttnPara
     o[3] = o[3] * a + (float)hc[3] * b;
     m_run = mn;
   }
-  if (wave > 0) {
-    s_o[wave - 1][0][lane] = m_run;
-    s_o[wave - 1][1][lane] = w_sum;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) s_o[wave - 1][2 + v][lane] = o[v];
-  }
-  __syncthreads();
   const int row = rb * kRows + rg * 32 + c32;
-  if (wave > 0 || row >= p.rows) return;
+  if constexpr (W == 4) {
+    if (wave > 0) {
+      s_o[wave - 1][0][lane] = m_run;
+      s_o[wave - 1][1][lane] = w_sum;
 #pragma unroll
-  for (int w = 0; w < 3; ++w) {
-    const float m2 = s_o[w][0][lane];
-    const float mn = fmaxf(m_run, m2);
-    const float ref = mn == -INFINITY ? 0.0f : mn;
-    const float a = exp2f(m_run - ref), b = exp2f(m2 - ref);
-    w_sum = w_sum * a + s_o[w][1][lane] * b;
+      for (int v = 0; v < 4; ++v) s_o[wave - 1][2 + v][lane] = o[v];
+    }
+    __syncthreads();
+    if (wave > 0) return;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) o[v] = o[v] * a + s_o[w][2 + v][lane] * b;
-    m_run = mn;
+    for (int w = 0; w < 3; ++w) {
+      const float m2 = s_o[w][0][lane];
+      const float mn = fmaxf(m_run, m2);
+      const float ref = mn == -INFINITY ? 0.0f : mn;
+      const float a = exp2f(m_run - ref), b = exp2f(m2 - ref);
+      w_sum = w_sum * a + s_o[w][1][lane] * b;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) o[v] = o[v] * a + s_o[w][2 + v][lane] * b;
+      m_run = mn;
+    }
   }
+  if (row >= p.rows) return;
   const int node = row % p.n;
   const int head = kvhead * p.group + row / p.n;
   const float inv = w_sum > 0.0f ? 1.0f / w_sum : 0.0f;
@@ -565,6 +573,18 @@ Split split_keys(int64_t seq_len, int64_t n, int64_t len) {
 int64_t groups_of(int64_t kvh, int64_t row_blocks, int64_t chunks) {
   return (kvh * chunks + 7) / 8 * 8 * row_blocks;
 }
+
+// Units of the combine that hold query rows.
+int64_t combine_units(int64_t kvh, int64_t rows) { return kvh * ((rows + 31) / 32) * 16; }
+
+// Waves per unit of the combine: from 1280 units on (five waves per CU) one wave
+// each keeps enough loads in flight, and four would add a barrier and four times
+// the workgroups.  Whole call, four waves against one, same box: 32 query over 32
+// KV heads, 256 nodes over 4096 / 8000 positions 37.1 / 59.5 -> 34.9 / 57.3 us, 100
+// over 2500 19.6 -> 18.3; 32 over 8, 100 nodes (1664 units) over 2500 20.3 -> 18.7,
+// 256 over 4096 35.8 -> 33.7; 64 over 8, 64 nodes over 4096 23.3 -> 22.3.  At 1024
+// units (32 over 8, 64 nodes over 4096) one wave took 20.0 against 18.7.
+int combine_waves(int64_t kvh, int64_t rows) { return combine_units(kvh, rows) >= 1280 ? 1 : 4; }
 
 // Planner cost of a split, in units of one 64-key stage of one workgroup:
 // the longest chunk's stages plus ~2 stages of workgroup prologue and
@@ -735,8 +755,10 @@ extern "C" int tm_tree_attention(const void* q, int64_t q_stride, const void* k_
   TM_HIP_CHECK_LAUNCH();
   if (pl.chunks > 1) {
     // KV heads x row blocks x four 32-row groups x 16 value groups
-    hipLaunchKernelGGL(tm_tree_attn_combine_kernel,
-                       dim3((unsigned)(kvh * pl.row_blocks * 4 * 16)), dim3(kThreads), 0,
+    const int64_t units = kvh * pl.row_blocks * 4 * 16;
+    const bool alone = combine_waves(kvh, p.rows) == 1;
+    hipLaunchKernelGGL(alone ? tm_tree_attn_combine_kernel<1> : tm_tree_attn_combine_kernel<4>,
+                       dim3((unsigned)(alone ? units / 4 : units)), dim3(kThreads), 0,
                        (hipStream_t)stream, p);
     TM_HIP_CHECK_LAUNCH();
   }
