@@ -594,10 +594,14 @@ int combine_waves(int64_t kvh, int64_t rows) { return combine_units(kvh, rows) >
 // loop over the chunks).  Fitted to measurements on MI355X at 1 .. 64 nodes and
 // 40 .. 8000 cached positions (32 query heads over 8 KV heads, 8 over 2), where
 // it picks the fastest chunk length of those tried or one within 4 % of it.
+// Chunks of one or two stages on shared CUs count as three: they load nothing
+// ahead (32 over 8, 72 / 90 nodes over 2500 positions: 21 chunks of two stages
+// 20.0 / 21.0 us, nine of five 17.7 / 18.5).
 double split_cost(const Split& sp, int64_t s_total, int64_t kvh, int64_t row_blocks) {
   const int64_t keys = sp.chunks > 1 ? sp.len : s_total;
-  const double stages = (double)((keys + kKeys - 1) / kKeys);
   const int64_t groups = groups_of(kvh, row_blocks, sp.chunks);
+  const double stages =
+      (double)std::max<int64_t>((keys + kKeys - 1) / kKeys, groups > kCUs ? 3 : 1);
   const double stretch = groups <= kCUs ? 1.0 : 0.8 * (double)((groups + kCUs - 1) / kCUs);
   const double combine = sp.chunks > 1 ? 1.6 + 0.04 * (double)sp.chunks : 0.0;
   return (stages + 2.0) * stretch + combine;
