@@ -384,6 +384,23 @@ def test_gemm_path_rule():
     assert m.uses_tiled_gemms(128, 8, 8, 1792)
 
 
+def test_gemm_path_rule_at_a_small_hidden_size():
+    """At H <= 1024 and I >= 3584 the tiled GEMMs run from 2 tokens, from 4 at H <= 512 or
+    17 .. 32 experts, from 6 at more; H = 0 (unknown) or larger keeps the row rules."""
+    from treemoe_spec_amd.kernels import op1_tree_moe as m
+
+    for e, h, first in ((8, 1024, 2), (8, 768, 2), (16, 1024, 2), (8, 512, 4), (8, 256, 4),
+                        (16, 512, 4), (17, 1024, 4), (32, 1024, 4), (32, 256, 4), (33, 1024, 6),
+                        (64, 512, 6)):
+        for budget in (2, e):
+            rows = 8 * min(budget, e) // 2        # tokens of the row rule at this width
+            for t in range(1, min(first, rows)):
+                assert not m.uses_tiled_gemms(t, budget, e, 3584, h), (t, e, h)
+        assert m.uses_tiled_gemms(first, e, e, 3584, h) and m.uses_tiled_gemms(first, e, e, 14336, h)
+        assert not m.uses_tiled_gemms(first, e, e, 3328, h)
+    assert not m.uses_tiled_gemms(8, 8, 8, 3584, 1280)
+    assert not m.uses_tiled_gemms(8, 8, 8, 3584)
+
 
 def test_tiled_gate_up_tile_rule():
     """The gate/up tile the library picks (named in bench lines): 256-row tiles

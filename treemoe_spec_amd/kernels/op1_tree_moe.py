@@ -70,24 +70,40 @@ TILED_MIN_ROWS_WIDE = 8       # .. or from this many when inter >= TILED_WIDE_IN
 TILED_WIDE_INTER = 3584
 
 # At a small hidden size the streaming kernels' work items are too short to
-# stream (gate/up: four K chunks, one per wave) and their latency shows, so the
-# tiled pair wins from two tokens on.  H=1024, I=3584, E=8, layer us, streaming /
-# tiled: B=8 T=1 26.8 / 27.7, T=2 36.0 / 30.7, T=4 51.6 / 38.0, T=24 57.5 / 42.1;
-# B=4 T=2 33.6 / 29.0, T=12 38.3 / 30.7; through the hook (routing in its own
-# launches) T=2 35.9 / 35.3, T=4 51.6 / 43.4.  H=4096, I=3584: T=4 111.4 / 110.8.
+# stream (gate/up: at most four K chunks, one per wave) and their latency shows,
+# so the tiled pair wins from a few tokens on, in an FFN wide enough to give it
+# column jobs.  How few: with the router's work (experts) and the launches
+# growing against the GEMMs it takes more rows.  Device us of a layer through the
+# hook, streaming / tiled, I=3584 (the forward call routes itself up to 16
+# experts and saves 5 us more):
+#   E=8   H=1024 T=2 33.1 / 32.4, T=4 47.3 / 39.5; H=768 T=2 30.2 / 29.7;
+#         H=512 T=2 26.7 / 27.2, T=4 35.7 / 31.4; H=256 T=3 26.5 / 27.4, T=4 30.0 / 27.9
+#   E=16  H=1024 T=2 40.0 / 38.0; H=512 T=2 31.5 / 31.9; H=256 T=3 31.4 / 31.9
+#   E=32  H=1024 T=3 54.2 / 55.8, T=4 61.2 / 58.6; H=256 T=2 34.9 / 36.8, T=4 42.1 / 39.9
+#   E=64  H=512 T=2 51.5 / 57.7, T=4 61.8 / 62.6, T=6 67.2 / 64.0
+# and at wider FFNs H=512, I=14336, E=8 T=3 54.5 / 55.3, T=4 61.9 / 60.9; above
+# the limit H=4096, I=3584, E=8 T=4 111.4 / 110.8.
 TILED_SMALL_HIDDEN = 1024
+
+
+def _small_hidden_tokens(num_experts: int, hidden: int) -> int:
+    """Tokens from which a layer of at most TILED_SMALL_HIDDEN takes the tiled GEMMs."""
+    if num_experts <= 16 and 2 * hidden > TILED_SMALL_HIDDEN:
+        return 2
+    return 4 if num_experts <= 32 else 6
 
 
 def uses_tiled_gemms(num_tokens: int, expert_budget: int, num_experts: int,
                      inter: int = 0, hidden: int = 0) -> bool:
     """True when the average rows per routed expert reach TILED_MIN_ROWS, or for
     an intermediate size of TILED_WIDE_INTER or more TILED_MIN_ROWS_WIDE, or
-    there two tokens where the hidden size (0: unknown) is at most
-    TILED_SMALL_HIDDEN."""
+    there a few tokens (_small_hidden_tokens) where the hidden size (0: unknown)
+    is at most TILED_SMALL_HIDDEN."""
     active = min(expert_budget, num_experts)
     if 2 * num_tokens >= TILED_MIN_ROWS * active:
         return True
-    if 0 < hidden <= TILED_SMALL_HIDDEN and inter >= TILED_WIDE_INTER and num_tokens >= 2:
+    if (0 < hidden <= TILED_SMALL_HIDDEN and inter >= TILED_WIDE_INTER
+            and num_tokens >= _small_hidden_tokens(num_experts, hidden)):
         return True
     return inter >= TILED_WIDE_INTER and 2 * num_tokens >= TILED_MIN_ROWS_WIDE * active
 
