@@ -309,7 +309,7 @@ def main():
     routed = bd.pop("self_routed")
     max_tiles = bd.pop("max_tiles")
     gemm1_kernel = (f"tm_prefill_gemm1{'_routed' if routed else ''}_kernel"
-                    f"<{m.tiled_gate_up_tile(t, e, max_tiles)}>" if tiled else "tm_gemm1_kernel")
+                    f"<{m.tiled_gate_up_tile(t, e, max_tiles, h, i)}>" if tiled else "tm_gemm1_kernel")
     # algorithmic bytes per launch: one read of the active experts' weights
     # (w1 + w3 for gemm1, w2 for gemm2) plus the activation rows in (x); the
     # h and fp32-partial workspaces are not counted

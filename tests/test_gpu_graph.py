@@ -67,6 +67,8 @@ def test_op1_graph_replays_equal_eager(path, t, budget, monkeypatch):
     m = _op1()
     monkeypatch.setattr(m, "TILED_MIN_ROWS", 1 << 30 if path == "stream" else 1)
     monkeypatch.setattr(m, "TILED_MIN_ROWS_WIDE", 1 << 30 if path == "stream" else 1)
+    if path == "stream":
+        monkeypatch.setattr(m, "TILED_SMALL_HIDDEN", 0)
     if path == "tiled_bucket":
         monkeypatch.setattr(m, "SELF_ROUTED_MAX_TOKENS", 0)
     e, h, i = (8, 512, 1024) if t <= 64 else (2, 512, 6144)

@@ -327,6 +327,8 @@ def _force_path(monkeypatch, path):
     m = _op1()
     monkeypatch.setattr(m, "TILED_MIN_ROWS", 1 << 30 if path == "stream" else 1)
     monkeypatch.setattr(m, "TILED_MIN_ROWS_WIDE", 1 << 30 if path == "stream" else 1)
+    if path == "stream":
+        monkeypatch.setattr(m, "TILED_SMALL_HIDDEN", 0)
     if path == "tiled_bucket":
         monkeypatch.setattr(m, "SELF_ROUTED_MAX_TOKENS", 0)
 

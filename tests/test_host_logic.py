@@ -403,9 +403,10 @@ def test_gemm_path_rule_at_a_small_hidden_size():
 
 
 def test_tiled_gate_up_tile_rule():
-    """The gate/up tile the library picks (named in bench lines): 256-row tiles
-    from 384 rows per expert, the 64-row decode tile when the tile list
-    leaves at most 16 rows per entry, else 128-row tiles."""
+    """The gate/up tile the library picks, by the name it has in the kernel's (bench lines):
+    256-row tiles from 112 rows per expert on where their jobs fill the GPU, the
+    64-row decode tile when the tile list leaves at most 16 rows per entry, else
+    128-row tiles."""
     from treemoe_spec_amd.kernels import op1_tree_moe as m
 
     def tiles(t, budget, e=8):
@@ -413,9 +414,24 @@ def test_tiled_gate_up_tile_rule():
 
     assert m.tiled_gate_up_tile(64, 8, tiles(64, 8)) == "Tile<64, 64, 3, 128, 256>"   # config 2
     assert m.tiled_gate_up_tile(64, 8, tiles(64, 4)) == "Tile<128, 64, 3>"            # config 3
-    assert m.tiled_gate_up_tile(2048, 8, tiles(2048, 8)) == "Tile<256, 32, 4>"        # config 5
+    assert m.tiled_gate_up_tile(2048, 8, tiles(2048, 8)) == "Tile<256, 64, 5, 256, 256>"  # config 5
     assert m.tiled_gate_up_tile(32, 8, tiles(32, 8)) == "Tile<64, 64, 3, 128, 256>"
     assert m.tiled_gate_up_tile(128, 8, tiles(128, 8)) == "Tile<128, 64, 3>"
+    # 112 rows per expert: T = 447 and 517; a narrow layer keeps the 128-row tile
+    assert m.tiled_gate_up_tile(447, 8, tiles(447, 8)) == "Tile<128, 64, 3>"
+    assert m.tiled_gate_up_tile(517, 8, tiles(517, 8)) == "Tile<256, 64, 5, 256, 256>"
+    assert m.tiled_gate_up_tile(517, 8, tiles(517, 8), 512, 2048) == "Tile<128, 64, 3>"
+
+
+def test_tile_names_are_those_of_the_kernels():
+    """The template arguments of the three tiles in op1_prefill.hip."""
+    import re
+    from pathlib import Path
+
+    from treemoe_spec_amd.kernels import op1_tree_moe as m
+
+    src = (Path(m.__file__).parents[1] / "csrc" / "op1_prefill.hip").read_text()
+    assert set(m._TILE_NAMES.values()) == set(re.findall(r"using Tile\w+ = (Tile<[^>]*>);", src))
 
 
 def test_bench_refuses_more_than_one_gpu():

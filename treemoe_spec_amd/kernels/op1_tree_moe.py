@@ -22,6 +22,7 @@ There is no CPU path: CPU tensors, other dtypes, or a missing library raise.
 
 from __future__ import annotations
 
+import ctypes
 import os
 
 import torch
@@ -108,18 +109,18 @@ def uses_tiled_gemms(num_tokens: int, expert_budget: int, num_experts: int,
     return inter >= TILED_WIDE_INTER and 2 * num_tokens >= TILED_MIN_ROWS_WIDE * active
 
 
-def tiled_gate_up_tile(num_tokens: int, num_experts: int, max_tiles: int) -> str:
-    """The tile tm_op1_prefill_gemm1 picks (the rule in op1_prefill.hip):
-    256-row tiles when the experts average 112 rows or more, the 64-row
-    decode tile when the tile list leaves at most 16 rows per entry, else
-    128-row tiles.  For naming kernels in measurements: the labels stay the same
-    from build to build, so the 256-row tile keeps the one it had with K steps
-    of 32 and four stages."""
-    if 2 * num_tokens >= 112 * num_experts:
-        return "Tile<256, 32, 4>"
-    if 2 * num_tokens <= 16 * max_tiles:
-        return "Tile<64, 64, 3, 128, 256>"
-    return "Tile<128, 64, 3>"
+_TILE_NAMES = {256: "Tile<256, 64, 5, 256, 256>", 128: "Tile<128, 64, 3>",
+               64: "Tile<64, 64, 3, 128, 256>"}
+
+
+def tiled_gate_up_tile(num_tokens: int, num_experts: int, max_tiles: int, hidden: int = 4096,
+                       inter: int = 14336) -> str:
+    """The tile tm_op1_prefill_gemm1 picks (tm_op1_prefill_tiles), as it stands
+    in the kernel's name.  For naming kernels in measurements."""
+    gate_up, down = ctypes.c_int64(), ctypes.c_int64()
+    call("tm_op1_prefill_tiles", max_tiles, 1, num_tokens, hidden, inter, num_experts,
+         ctypes.byref(gate_up), ctypes.byref(down))
+    return _TILE_NAMES[gate_up.value]
 
 
 def _split_for(inter: int) -> int:
