@@ -109,12 +109,7 @@ struct Top2 {
 // and never read back here.  So the phases are separated by LDS-only barriers:
 // __syncthreads() would also wait for the phase's global stores to complete
 // (its workgroup release fence), measured at 0.5-1 us per phase.
-//
-// WRITE = false computes the per-expert counts (sh.count), the compact
-// offsets (sh.offset) and the compact order (sh.sorted) in LDS only, for a
-// GEMM workgroup that needs its own rows; WRITE = true also writes every
-// routing output to global memory.
-template <int NT, class SH, bool WRITE>
+template <int NT, class SH>
 __device__ void bucket_phases(const BucketArgs& a, SH& sh) {
   constexpr int NW = NT / 64;
   const int tid = threadIdx.x;
@@ -143,8 +138,7 @@ __device__ void bucket_phases(const BucketArgs& a, SH& sh) {
   }
 #pragma unroll 8
   for (int t = tid; t < T; t += NT) sh.accept[t] = a.accept[t];
-  if constexpr (WRITE)
-    for (int b = tid; b < a.max_blocks; b += NT) sh.owner[b] = -1;
+  for (int b = tid; b < a.max_blocks; b += NT) sh.owner[b] = -1;
   tm_lds_barrier();
   const float* G = staged ? sh.gates : a.gates;
 
@@ -180,7 +174,7 @@ __device__ void bucket_phases(const BucketArgs& a, SH& sh) {
     if (lane == 0) {
       sh.demand[e] = acc;
       sh.crit[e] = crit;
-      if constexpr (WRITE) a.demand_out[e] = acc;
+      a.demand_out[e] = acc;
     }
   }
   tm_lds_barrier();
@@ -227,16 +221,14 @@ __device__ void bucket_phases(const BucketArgs& a, SH& sh) {
     } else {
       for (int e = 0; e < E; ++e) r.offer(((keep >> e) & 1ull) ? g[e] : 0.0f, e);
     }
-    if constexpr (WRITE) {
-      const float s = r.g1 + r.g2;
-      float tg1 = r.g1 / s;
-      float tg2 = r.g2 / s;
-      if (sh.accept[t] < a.tau) { tg1 = 1.0f; tg2 = 0.0f; }
-      a.topk_ids[2 * t] = r.i1;
-      a.topk_ids[2 * t + 1] = r.i2;
-      a.gates_flat[2 * t] = tg1;
-      a.gates_flat[2 * t + 1] = tg2;
-    }
+    const float s = r.g1 + r.g2;
+    float tg1 = r.g1 / s;
+    float tg2 = r.g2 / s;
+    if (sh.accept[t] < a.tau) { tg1 = 1.0f; tg2 = 0.0f; }
+    a.topk_ids[2 * t] = r.i1;
+    a.topk_ids[2 * t + 1] = r.i2;
+    a.gates_flat[2 * t] = tg1;
+    a.gates_flat[2 * t + 1] = tg2;
     sh.fe[2 * t] = (uint8_t)r.i1;  // the critical-path use of fe ended at an earlier barrier
     sh.fe[2 * t + 1] = (uint8_t)r.i2;
   }
@@ -256,17 +248,15 @@ __device__ void bucket_phases(const BucketArgs& a, SH& sh) {
     if (s < nslot) sh.inrank[s] = (uint8_t)inrank;
   }
   tm_lds_barrier();
-  // 4b. exclusive scan over chunks (slot order) per expert; chunks q and q+64
-  //     of one expert sit in lane q of the wave that owns the expert.
+  // 4b. exclusive scan over chunks (slot order) per expert; chunk q of one expert
+  //     sits in lane q of the wave that owns the expert.
+  static_assert(SH::kMaxChunks <= 64, "one chunk per lane");
   for (int e = wave; e < E; e += NW) {
-    const int v0 = (lane < nchunk) ? (int)sh.cnt[lane * TM_MAX_EXPERTS + e] : 0;
-    const int v1 = (lane + 64 < nchunk) ? (int)sh.cnt[(lane + 64) * TM_MAX_EXPERTS + e] : 0;
-    int tot0, tot1;
-    const int x0 = wave_exclusive_scan(v0, lane, &tot0);
-    const int x1 = wave_exclusive_scan(v1, lane, &tot1);
-    if (lane < nchunk) sh.cnt[lane * TM_MAX_EXPERTS + e] = (uint16_t)x0;
-    if (lane + 64 < nchunk) sh.cnt[(lane + 64) * TM_MAX_EXPERTS + e] = (uint16_t)(tot0 + x1);
-    if (lane == 0) sh.count[e] = tot0 + tot1;
+    const int v = (lane < nchunk) ? (int)sh.cnt[lane * TM_MAX_EXPERTS + e] : 0;
+    int tot;
+    const int x = wave_exclusive_scan(v, lane, &tot);
+    if (lane < nchunk) sh.cnt[lane * TM_MAX_EXPERTS + e] = (uint16_t)x;
+    if (lane == 0) sh.count[e] = tot;
   }
   tm_lds_barrier();
   // 4c. block layout (reference), compact offsets and GEMM tiles (wave 0,
@@ -277,34 +267,32 @@ __device__ void bucket_phases(const BucketArgs& a, SH& sh) {
     const int off = wave_exclusive_scan(c, lane, &tot_off);
     if (lane < E) sh.offset[lane] = off;
     if (lane == 0) sh.offset[E] = tot_off;
-    if constexpr (WRITE) {
-      const int nb = (c + a.BM - 1) / a.BM;
-      const int nt = (c + TM_GEMM_TILE_M - 1) / TM_GEMM_TILE_M;
-      int tot_blk, tot_tiles;
-      const int bs = wave_exclusive_scan(nb, lane, &tot_blk);
-      const int ts = wave_exclusive_scan(nt, lane, &tot_tiles);
-      if (lane < E) {
-        sh.block_start[lane] = bs;
-        sh.nblocks[lane] = nb;
-        a.expert_offsets[lane] = off;
-        for (int b = bs; b < min(bs + nb, a.max_blocks); ++b) sh.owner[b] = (int16_t)lane;
-        for (int k = 0; k < nt; ++k) {
-          const int j = ts + k;
-          if (j < a.max_tiles) {
-            a.tiles[4 * j + 0] = lane;
-            a.tiles[4 * j + 1] = off + k * TM_GEMM_TILE_M;
-            a.tiles[4 * j + 2] = min(TM_GEMM_TILE_M, c - k * TM_GEMM_TILE_M);
-            a.tiles[4 * j + 3] = 0;
-          }
+    const int nb = (c + a.BM - 1) / a.BM;
+    const int nt = (c + TM_GEMM_TILE_M - 1) / TM_GEMM_TILE_M;
+    int tot_blk, tot_tiles;
+    const int bs = wave_exclusive_scan(nb, lane, &tot_blk);
+    const int ts = wave_exclusive_scan(nt, lane, &tot_tiles);
+    if (lane < E) {
+      sh.block_start[lane] = bs;
+      sh.nblocks[lane] = nb;
+      a.expert_offsets[lane] = off;
+      for (int b = bs; b < min(bs + nb, a.max_blocks); ++b) sh.owner[b] = (int16_t)lane;
+      for (int k = 0; k < nt; ++k) {
+        const int j = ts + k;
+        if (j < a.max_tiles) {
+          a.tiles[4 * j + 0] = lane;
+          a.tiles[4 * j + 1] = off + k * TM_GEMM_TILE_M;
+          a.tiles[4 * j + 2] = min(TM_GEMM_TILE_M, c - k * TM_GEMM_TILE_M);
+          a.tiles[4 * j + 3] = 0;
         }
       }
-      if (lane == 0) a.expert_offsets[E] = tot_off;
-      for (int j = tot_tiles + lane; j < a.max_tiles; j += 64) {
-        a.tiles[4 * j + 0] = -1;
-        a.tiles[4 * j + 1] = 0;
-        a.tiles[4 * j + 2] = 0;
-        a.tiles[4 * j + 3] = 0;
-      }
+    }
+    if (lane == 0) a.expert_offsets[E] = tot_off;
+    for (int j = tot_tiles + lane; j < a.max_tiles; j += 64) {
+      a.tiles[4 * j + 0] = -1;
+      a.tiles[4 * j + 1] = 0;
+      a.tiles[4 * j + 2] = 0;
+      a.tiles[4 * j + 3] = 0;
     }
   }
   tm_lds_barrier();
@@ -313,29 +301,23 @@ __device__ void bucket_phases(const BucketArgs& a, SH& sh) {
     const int fe = sh.fe[s];
     const int rank = (int)sh.cnt[(s >> 6) * TM_MAX_EXPERTS + fe] + (int)sh.inrank[s];
     const int pos = sh.offset[fe] + rank;
-    if constexpr (WRITE) {
-      a.slot_to_row[s] = sh.block_start[fe] * a.BM + rank;
-      a.sorted_slots[pos] = s;
-      a.slot_pos[s] = pos;
-    }
+    a.slot_to_row[s] = sh.block_start[fe] * a.BM + rank;
+    a.sorted_slots[pos] = s;
+    a.slot_pos[s] = pos;
     sh.sorted[pos] = (uint16_t)s;
   }
-  if constexpr (WRITE) {
-    for (int b = tid; b < a.max_blocks; b += NT) a.block_expert_ids[b] = sh.owner[b];
-  }
+  for (int b = tid; b < a.max_blocks; b += NT) a.block_expert_ids[b] = sh.owner[b];
   tm_lds_barrier();
   // 4e. padded rows: row i of block b holds the (i - first row of the owner)-th
   //     slot of the owning expert, or -1 past its count or in an unused block.
-  if constexpr (WRITE) {
-    for (int i = tid; i < padded_rows; i += NT) {
-      const int e = sh.owner[i / a.BM];
-      int64_t slot = -1;
-      if (e >= 0) {
-        const int rank = i - sh.block_start[e] * a.BM;
-        if (rank < sh.count[e]) slot = sh.sorted[sh.offset[e] + rank];
-      }
-      a.padded_slots[i] = slot;
+  for (int i = tid; i < padded_rows; i += NT) {
+    const int e = sh.owner[i / a.BM];
+    int64_t slot = -1;
+    if (e >= 0) {
+      const int rank = i - sh.block_start[e] * a.BM;
+      if (rank < sh.count[e]) slot = sh.sorted[sh.offset[e] + rank];
     }
+    a.padded_slots[i] = slot;
   }
 }
 

@@ -909,7 +909,7 @@ tm_prefill_gemm1_routed_kernel(const uint16_t* __restrict__ x, const uint16_t* _
   static_assert(sizeof(RvShared) <= C::BUF, "the routing writer uses the first stage");
   const int L = (int)blockIdx.x;
   if (L < kRvLeaders) {
-    if (L == 0) tmb::bucket_phases<C::NT, RvShared, true>(ra, *reinterpret_cast<RvShared*>(s0));
+    if (L == 0) tmb::bucket_phases<C::NT, RvShared>(ra, *reinterpret_cast<RvShared*>(s0));
     return;
   }
   int e, p0, rows, m0, cb;

@@ -26,7 +26,10 @@ constexpr int kWaves = kThreads / 64;
 // From this many tokens the bucketing is spread over the chip; below, one
 // workgroup keeps every per-slot intermediate in LDS.
 constexpr int kSpreadMinTokens = 1024;
-// Up to this many tokens the caller's padded rows are bounded by kMaxPaddedRows.
+// Up to this many tokens more than kMaxPaddedRows padded rows are refused: the
+// one-workgroup kernel's block table, and above kSpreadMinTokens a limit of the
+// entry points that no call with its routing's own max_blocks reaches (2 T rows
+// in at most 64 experts).
 constexpr int kFewTokens = 4096;
 constexpr int kMaxPaddedRows = 16384;
 // Tokens from which the row router runs: its per-workgroup W_g copy costs
@@ -274,7 +277,7 @@ tm_route_fused_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict
 
 __global__ void __launch_bounds__(kThreads) tm_bucket_kernel(BucketArgs args) {
   __shared__ __attribute__((aligned(16))) BucketShared sh;
-  tmb::bucket_phases<kThreads, BucketShared, true>(args, sh);
+  tmb::bucket_phases<kThreads, BucketShared>(args, sh);
 }
 
 // ------------------------------------------------------ many tokens --
@@ -603,7 +606,7 @@ int check_bucket_args(int64_t T, int64_t E, int64_t budget, int objective, int64
 void launch_bucket(const BucketArgs& a, hipStream_t stream) {
   if (a.T <= kWaveMaxTokens && a.E <= kWaveMaxExperts) {
     hipLaunchKernelGGL(tm_bucket_wave_kernel, dim3(1), dim3(kWaveThreads), 0, stream, a);
-  } else if (a.T < kSpreadMinTokens && a.max_blocks * a.BM <= kMaxPaddedRows) {
+  } else if (a.T < kSpreadMinTokens) {
     hipLaunchKernelGGL(tm_bucket_kernel, dim3(1), dim3(kThreads), 0, stream, a);
   } else {
     const int groups = (a.T + kSpreadThreads - 1) / kSpreadThreads;
