@@ -90,6 +90,68 @@ def test_tile256_gemms_match_float64(steps):
             assert torch.all((out[s, r] - ref).abs() <= tol), (steps, COUNTS[k], s)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("counts,masked,i", [
+    ([0, 300, 0, 257, 1, 0, 512, 64, 0, 130, 0], (), 4096),    # empty first, last and between
+    ([200, 300, 256, 257, 1, 255, 513, 64], (0, 2, 7), 3072),  # masked, as exclude_experts does
+    ([0, 400, 401, 0, 399, 400], (2,), 3072),
+])
+def test_tile256_empty_and_masked_experts(counts, masked, i, dtype):
+    """Empty experts have no M-tiles; a masked one keeps its tiles in the job order and leaves its
+    rows of h and y alone."""
+    from treemoe_spec_amd import _capi
+
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(sum(counts))
+    e, rows = len(counts), sum(counts)
+    t, h, split = rows // 2, 256, 2
+    offsets, tiles = [0], []
+    for k, c in enumerate(counts):
+        tiles += [[-1 if k in masked else k, offsets[k] + r0, min(64, c - r0), 0]
+                  for r0 in range(0, c, 64)]
+        offsets.append(offsets[-1] + c)
+    nt = len(tiles)
+    assert rows % 2 == 0 and _tiles(nt, 1, t, h, i, e)[0] == 256
+    assert _tiles(nt, split, t, i, 2 * h, e)[1] == 256
+    print(f"tile256 empty/masked {counts} {masked} {dtype}", flush=True)
+    code = _capi.TM_DTYPE_BF16 if dtype == torch.bfloat16 else _capi.TM_DTYPE_F16
+    half_ulp = torch.finfo(dtype).eps / 2
+    as_dev = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    slots = torch.randperm(rows, generator=g).to(torch.int32)
+    draw = lambda *s: torch.randn(*s, generator=g).to(dtype)
+    x, w1, w3 = draw(t, h), draw(e, i, h) * 0.1, draw(e, i, h) * 0.1
+    xd, w1d, w3d, sd, od, td = (x.to(dev), w1.to(dev), w3.to(dev), slots.to(dev),
+                                as_dev(offsets), as_dev(tiles))
+    hd = torch.full((rows, i), 7.0, dtype=dtype, device=dev)
+    st = _capi.stream_of(dev)
+    _capi.call("tm_op1_prefill_gemm1", xd.data_ptr(), w1d.data_ptr(), w3d.data_ptr(),
+               hd.data_ptr(), sd.data_ptr(), od.data_ptr(), td.data_ptr(), nt, t, h, i, e, code, st)
+    out = hd.double().cpu()
+    # down: i output columns, two segments of K = 256
+    hm, w2, gates = draw(rows, 2 * h), draw(e, i, 2 * h) * 0.1, torch.rand(rows, generator=g)
+    hmd, w2d, gd = hm.to(dev), w2.to(dev), gates.to(dev)
+    y = torch.full((split, rows, i), 7.0, device=dev)
+    _capi.call("tm_op1_prefill_gemm2", hmd.data_ptr(), w2d.data_ptr(), y.data_ptr(),
+               gd.data_ptr(), sd.data_ptr(), od.data_ptr(), td.data_ptr(), nt, split, t, i, 2 * h,
+               e, code, st)
+    yo = y.double().cpu()
+    for k in range(e):
+        r = slice(offsets[k], offsets[k + 1])
+        if k in masked:
+            assert torch.all(out[r] == 7.0) and torch.all(yo[:, r] == 7.0), k
+            continue
+        xf = x[slots[r].long() >> 1].double()
+        a, b = xf @ w1[k].double().T, xf @ w3[k].double().T
+        ref = a * torch.sigmoid(a) * b
+        tol = 2 * half_ulp * ref.abs() + 1e-5 * (1.0 + a.abs()) * (1.0 + b.abs())
+        assert torch.all((out[r] - ref).abs() <= tol), k
+        for s in range(split):
+            p, w = hm[r, s * h:(s + 1) * h].double(), w2[k, :, s * h:(s + 1) * h].double()
+            gate = gates[slots[r].long()].double()[:, None]
+            ref, mag = gate * (p @ w.T), gate * (p.abs() @ w.abs().T)
+            assert torch.all((yo[s, r] - ref).abs() <= (h + 2) * 2.0 ** -24 * mag), (k, s)
+
+
 @pytest.mark.parametrize("counts", [[16] * 8, [1, 15, 64, 65, 3, 0, 28, 0], [2, 2], [128, 0, 0, 0]])
 def test_narrow_down_tile_matches_float64(counts):
     """Down with too few 128-row jobs for the chip (64-row tiles, 128 columns)."""
