@@ -236,3 +236,22 @@ def test_cpython_binding_loads_and_checks_arguments():
     for name in ("argmax_walk", "kv_commit"):
         with pytest.raises(TypeError):
             getattr(_tmfast, name)(1, 2, 3)
+
+
+def test_library_override_reaches_every_call(tmp_path):
+    """With TREEMOE_AMD_LIB naming another library, no call goes through the CPython binding,
+    which is linked to the one beside it."""
+    import os
+    import shutil
+    import subprocess
+    import sys
+
+    from treemoe_spec_amd import _capi
+
+    other = shutil.copy(_capi._LIB_PATH, tmp_path / "lib.so")
+    code = ("from treemoe_spec_amd.kernels import op4_commit, tree_attention\n"
+            "print(tree_attention._fast, op4_commit._fast)")
+    env = {**os.environ, "TREEMOE_AMD_LIB": str(other)}
+    out = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env=env, check=True,
+                         capture_output=True, text=True).stdout
+    assert out.split() == ["None", "None"]

@@ -78,6 +78,18 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+def fast_binding():
+    """The CPython binding of the per-step entry points, or None where it is not
+    built or TREEMOE_AMD_LIB names a library other than the one it is linked to."""
+    if _LIB_PATH.resolve() != Path(__file__).resolve().parent / "libtreemoe_amd.so":
+        return None
+    try:
+        from treemoe_spec_amd import _tmfast
+    except ImportError:
+        return None
+    return _tmfast
+
+
 def check(rc: int, what: str) -> None:
     if rc != 0:
         msg = lib().tm_status_string(rc).decode()

@@ -47,10 +47,7 @@ from treemoe_spec_amd.kv_cache import device_tables_of, scratch_pages_of
 # The per-step greedy path calls the C ABI through the CPython binding when it
 # is built (one Python-to-C transition per entry point instead of ctypes'
 # per-argument conversions); the ctypes binding serves every other call.
-try:
-    from treemoe_spec_amd import _tmfast as _fast
-except ImportError:  # not built: the ctypes binding is used
-    _fast = None
+_fast = _capi.fast_binding()
 
 
 @dataclass

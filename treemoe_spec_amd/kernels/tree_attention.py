@@ -33,10 +33,7 @@ from treemoe_spec_amd.kv_cache import device_tables_of, scratch_pages_of
 # instead of through a tensor view.  Host time of a call 14-17 -> 8 us, which
 # is what bounded the short contexts (27 nodes over 333 positions: 10.5 us on
 # the device).
-try:
-    from treemoe_spec_amd import _tmfast as _fast
-except ImportError:  # not built: the ctypes binding is used
-    _fast = None
+_fast = _capi.fast_binding()
 
 _mask_cache: dict = {}
 _CACHE_ENTRIES = 16
