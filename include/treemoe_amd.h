@@ -92,7 +92,9 @@ int tm_op1_router_gates(const void* x, const void* wg, int64_t T, int64_t H,
                         int64_t E, float* gates, int dtype, void* stream);
 
 /*
- * Budget routing + stable (expert, DFS) bucketing in one workgroup.
+ * Budget routing + stable (expert, DFS) bucketing: one launch of one workgroup
+ * below 1024 tokens, from there two or three launches spread over the GPU, in
+ * which slot_to_row holds intermediate values until the last one writes it.
  * Replaces `_budget_bucket_fused_kernel` (treemoe/kernels/op1_tree_moe.py:159-297)
  * and its torch fallback `route_and_bucket` (:81-149); semantics of
  * `budget_route_ref` (treemoe/ref/tree_moe_ref.py:14-67) and
@@ -122,10 +124,11 @@ int tm_op1_route_bucket(const float* gates, const float* accept, int64_t T,
                         int32_t* slot_pos, int32_t* tiles, void* stream);
 
 /*
- * Router + budget routing + bucketing in one call (two launches on `stream`:
- * one workgroup per token computes that token's gates exactly as
- * tm_op1_router_gates, then one workgroup buckets all tokens exactly as
- * tm_op1_route_bucket).  Replaces the reference's router
+ * Router + budget routing + bucketing in one call: the gates exactly as
+ * tm_op1_router_gates computes them, then the bucketing exactly as
+ * tm_op1_route_bucket.  One launch on `stream` for at most 16 logits (T * E) of
+ * at most 8 experts, else the router's and the bucketing's.  Replaces the
+ * reference's router
  * (op1_tree_moe.py:676-677) plus `_budget_bucket_fused_kernel` (:159-297) as
  * launched by `route_experts` (:641-708).  Arguments and outputs are the union
  * of the two entry points above; gates [T, E] fp32 is written too.

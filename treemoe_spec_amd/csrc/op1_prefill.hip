@@ -465,10 +465,11 @@ __device__ __forceinline__ int frag_off(int lane, int s) {
 // workgroups of the XCD share, most of one.  A wave reads 256 fragment rows
 // per 128 x 128 outputs where two waves of 128 x 64 read 384: a third less LDS
 // traffic.
-// What bounds it: the card's power.  Under this loop the clock falls from 2.4
-// to 1.5-1.8 GHz, so time follows the energy of a flop: the operand bytes moved
-// (hence one wave per SIMD with large tiles and whole 128-byte lines per load)
-// as much as the stalls.  H = 4096, I = 14336, E = 8, same box, against the
+// What bounds it: operands and the clock.  Under this loop the clock falls from 2.4
+// to 1.8-1.95 GHz (GRBM_GUI_ACTIVE over the dispatches' time, T = 2048 skewed), the
+// matrix cores are busy 53-58 % of its cycles and the waves wait 55-62 % of theirs,
+// so the operand bytes moved (hence one wave per SIMD with large tiles and whole
+// 128-byte lines per load) count as much as the stalls.  H = 4096, I = 14336, E = 8, same box, against the
 // 8-wave loop of two 4-wave halves half a step apart with K steps of 32 (down:
 // 128-row tiles, steps of 64) that it replaces: T = 6011 gate/up 2560 -> 2200 us
 // (1.28 PFLOP/s), down 1437 -> 1188; T = 2048 skewed 995 -> 858 and 573 -> 481;

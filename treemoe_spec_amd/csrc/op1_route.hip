@@ -298,7 +298,10 @@ __global__ void __launch_bounds__(kThreads) tm_bucket_kernel(BucketArgs args) {
 // path, against one workgroup (above 4096 tokens through the output buffers):
 // T = 517 17.6 -> 16.6 / 20.5 -> 21.4 us, T = 1000 21.9 -> 18.7 / 21.9 -> 22.0,
 // T = 1500 27.4 -> 20.5 / 32.7 -> 25.3, T = 2048 31.7 -> 21.8 / 38.7 -> 26.7, T =
-// 6011 113 -> 42 / 148 -> 49; hence kSpreadMinTokens = 1024.
+// 6011 113 -> 42 / 148 -> 49; E = 64 T = 1024 97 -> 64 / 125 -> 104, T = 2048 182 -> 89 /
+// 235 -> 161; hence kSpreadMinTokens = 1024.  (Device times.  A stand-alone
+// route_and_bucket of 8 experts at 1024 .. 1500 tokens is bound by the host, which
+// pays 2.3 us per launch: 26.8 -> 28.5-29.8 us with a budget of 8.)
 constexpr int kSpreadThreads = 512;
 constexpr int kSpreadWaves = kSpreadThreads / 64;
 constexpr int kDemandTile = 8192;  // products staged in LDS at a time

@@ -6,7 +6,8 @@ Same Python surface as the reference module treemoe/kernels/op1_tree_moe.py
 work runs in libtreemoe_amd.so:
 
   routing      tm_op1_route          router (bf16 logits, fp32 softmax), then
-                                     budget routing + bucketing (two launches);
+                                     budget routing + bucketing (one to four
+                                     launches, by tokens and experts);
                                      at few tokens on the tiled path the
                                      bucketing runs inside the gate/up launch
                                      (tm_op1_prefill_gemm1_routed)
