@@ -308,8 +308,10 @@ def main():
     tiled = bd.pop("tiled")
     routed = bd.pop("self_routed")
     max_tiles = bd.pop("max_tiles")
-    gemm1_kernel = (f"tm_prefill_gemm1{'_routed' if routed else ''}_kernel"
-                    f"<{m.tiled_gate_up_tile(t, e, max_tiles, h, i)}>" if tiled else "tm_gemm1_kernel")
+    gemm1_kernel = "tm_gemm1_kernel"
+    if tiled:
+        gemm1_kernel = (f"tm_prefill_gemm1{'_routed' if routed else ''}_kernel"
+                        f"<{m.tiled_gate_up_tile(t, e, max_tiles, h, i)}>")
     # algorithmic bytes per launch: one read of the active experts' weights
     # (w1 + w3 for gemm1, w2 for gemm2) plus the activation rows in (x); the
     # h and fp32-partial workspaces are not counted

@@ -234,8 +234,9 @@ int tm_op1_prefill_gemm1_routed(const void* x, const void* w1, const void* w3, v
 
 /*
  * Down projection for many rows per expert, MFMA-tiled over 256 or 128 rows x
- * 256 output columns, or 64 rows x 128 (tm_op1_prefill_tiles); the prefill counterpart of tm_op1_gemm2 (reference
- * `_moe_gemm2_det_kernel`, treemoe/kernels/op1_tree_moe.py:447-509):
+ * 256 output columns, or 64 rows x 128 (tm_op1_prefill_tiles); the prefill
+ * counterpart of tm_op1_gemm2 (reference `_moe_gemm2_det_kernel`,
+ * treemoe/kernels/op1_tree_moe.py:447-509):
  *   y[s, p, n] = gates_flat[sorted_slots[p]] * sum_{k in segment s} h[p, k] w2[e, n, k]
  * with h row-major [2T, I] from tm_op1_prefill_gemm1 and y [split, 2T, H] fp32
  * in the layout tm_op1_combine reads; masked experts (as in

@@ -396,7 +396,8 @@ def test_gemm_path_rule_at_a_small_hidden_size():
             rows = 8 * min(budget, e) // 2        # tokens of the row rule at this width
             for t in range(1, min(first, rows)):
                 assert not m.uses_tiled_gemms(t, budget, e, 3584, h), (t, e, h)
-        assert m.uses_tiled_gemms(first, e, e, 3584, h) and m.uses_tiled_gemms(first, e, e, 14336, h)
+        assert m.uses_tiled_gemms(first, e, e, 3584, h)
+        assert m.uses_tiled_gemms(first, e, e, 14336, h)
         assert not m.uses_tiled_gemms(first, e, e, 3328, h)
     assert not m.uses_tiled_gemms(8, 8, 8, 3584, 1280)
     assert not m.uses_tiled_gemms(8, 8, 8, 3584)

@@ -469,12 +469,14 @@ __device__ __forceinline__ int frag_off(int lane, int s) {
 // to 1.8-1.95 GHz (GRBM_GUI_ACTIVE over the dispatches' time, T = 2048 skewed), the
 // matrix cores are busy 53-58 % of its cycles and the waves wait 55-62 % of theirs,
 // so the operand bytes moved (hence one wave per SIMD with large tiles and whole
-// 128-byte lines per load) count as much as the stalls.  H = 4096, I = 14336, E = 8, same box, against the
-// 8-wave loop of two 4-wave halves half a step apart with K steps of 32 (down:
-// 128-row tiles, steps of 64) that it replaces: T = 6011 gate/up 2560 -> 2200 us
-// (1.28 PFLOP/s), down 1437 -> 1188; T = 2048 skewed 995 -> 858 and 573 -> 481;
-// T = 517, on 128-row tiles before, 430 -> 355 and 262 -> 166.  The same loop
-// with K steps of 32 in four stages took 2410 and 1340 us at T = 6011.
+// 128-byte lines per load) count as much as the stalls.  H = 4096, I = 14336,
+// E = 8, same box, against the 8-wave loop of two 4-wave halves half a step apart
+// with K steps of 32 (down: 128-row tiles, steps of 64) that it replaces, gate/up
+// with SwiGLU by a reciprocal (its division adds 1.5 %, T = 6011 2258 -> 2293 us on
+// a slower box): T = 6011 gate/up 2560 -> 2200 us, down 1437 -> 1188; T = 2048
+// skewed 995 -> 858 and 573 -> 481; T = 517, on 128-row tiles before, 430 -> 355 and
+// 262 -> 166.  The same loop with K steps of 32 in four stages took 2410 and 1340 us
+// at T = 6011.
 template <class C, int M, int DT, bool NTB>
 struct PipeLoop {
   static constexpr int NJ = C::NJ, AL = C::ALD, BL = C::BLD;
